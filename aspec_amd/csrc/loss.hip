@@ -5,8 +5,8 @@
 //   row walk (V % 8 == 0, V <= 512*8*8): one 512-thread workgroup per CU walks the rows; each row
 //   of draft and teacher logits is read from HBM exactly once into registers while the previous
 //   row is reduced (max / sum / |p - q| / sign masses);
-//   streaming path (any V): one 256-thread workgroup per row, element loads, the rows re-read
-//   from cache per pass.
+//   streaming path (any V, any alignment): one workgroup per row, two passes over the row in
+//   16-byte chunks.
 // Backward: elementwise over rows x V from the saved per-row statistics (one read of x and y,
 // one write of dx).
 //
@@ -92,14 +92,6 @@ __device__ __forceinline__ float scalar_read_bf16(const uint16_t* p) {
   return __uint_as_float((a & 2) ? (w & 0xffff0000u) : (w << 16));
 }
 
-// Masses of p against q: accumulates |p-q| and p split by sign(p-q) (tiled_l1.py:76-92).
-__device__ __forceinline__ void l1_terms(float p, float q, float& l1, float& pos, float& neg, float& zero) {
-  l1 += fabsf(p - q);
-  if (p > q) pos += p;
-  else if (p < q) neg += p;
-  else zero += p;
-}
-
 // log2-domain exponent of a logit against its row maximum: p = exp2(v*log2e - max*log2e) / sum.
 // The forward and backward kernels evaluate it with this one formula, so they classify p against
 // q identically, and identical draft/teacher rows give bitwise equal probabilities.
@@ -147,6 +139,27 @@ __device__ __forceinline__ void block_max_sum(float (&m)[NP], float (&s)[NP], fl
 __device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
+// Eight consecutive bf16 as one 16-byte access at any 2-byte alignment, and the first n of them
+// element by element (the rest 0).
+typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t ChunkWords;
+__device__ __forceinline__ uint4 load_chunk(const uint16_t* p) {
+  const u32x4 v = *(const __attribute__((address_space(1))) ChunkWords*)(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void store_chunk(uint16_t* p, const uint4& v) {
+  *(__attribute__((address_space(1))) ChunkWords*)(p) = u32x4{v.x, v.y, v.z, v.w};
+}
+__device__ __forceinline__ uint4 load_part(const uint16_t* p, int n) {
+  uint32_t w[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t lo = 2 * k < n ? p[2 * k] : 0u;
+    const uint32_t hi = 2 * k + 1 < n ? p[2 * k + 1] : 0u;
+    w[k] = lo | (hi << 16);
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 constexpr int kWalkThreads = 512;  // threads of the persistent row walk (8 waves, 2 per SIMD)
 // Eight bf16 -inf: what the row walk's lanes past the end of a row load.
 __device__ const uint4 kNegInfChunk = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
@@ -169,6 +182,13 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
 __device__ __forceinline__ float min_abs_raw(float a, float b) {
   float r;
   asm("v_min_f32_e64 %0, %1, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// min(a, |b|, |c|), likewise.
+__device__ __forceinline__ float min3_abs_raw(float a, float b, float c) {
+  float r;
+  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
 
@@ -510,55 +530,201 @@ loss_fwd_persistent(LossArgs args) {
   }
 }
 
-// Any vocabulary size: element loads, three passes over the (cache-resident) row.
-__global__ void __launch_bounds__(256) loss_fwd_streaming(LossArgs a) {
+// Rows the walk does not take (V > 32768, V % 8 != 0, rows off 16-byte alignment): one workgroup
+// per row, two passes over it in chunks of eight logits. Pass 1 keeps each thread's running maximum
+// and sum (rescaled when a chunk raises the maximum) and the chunk that holds its maximum; pass 2
+// forms p and q from the row's statistics and sums the masses, last chunks first: those are still
+// in the L2.
+//
+// A chunk starts at a multiple of eight logits of its row, so at any 2-byte address when V % 8 != 0:
+// its load is one 16-byte access all the same (global memory takes any alignment on this target).
+//
+// What bounds it: both passes' reads. A 151936-token row and its teacher are 608 KB, more than a CU's
+// registers and LDS hold, so they are read twice; at 2048 rows against 1024 teacher rows the two
+// passes move 2.5 GB past the L2 in 395-420 us (6 TB/s; the previous kernel, element loads in three
+// passes, took 1467 us). Per logit pair pass 1 costs about 12 VALU slots and pass 2 16. Kept: two
+// chunks in flight per thread (one or three measured the same) and 512 threads (1024: 483 us at
+// 2048 rows and no faster at 64 rows; 256: the same at 2048 rows, 57 against 41 us at 64).
+template <int THREADS, bool HAS_Y>
+__global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
   __shared__ float scratch[4 * 32];
+  __shared__ uint32_t keys[THREADS / 64];
   const int64_t row = blockIdx.x;
-  const bool has_y = a.y != nullptr;
+  constexpr bool has_y = HAS_Y;
   const int64_t trow = has_y ? teacher_row(a, row) : 0;
-  const uint16_t* xr = a.x + row * a.V;
-  const uint16_t* yr = has_y && trow >= 0 ? a.y + trow * a.V : nullptr;
-  float m[2] = {-INFINITY, -INFINITY};
-  for (int64_t i = threadIdx.x; i < a.V; i += blockDim.x) {
-    m[0] = fmaxf(m[0], bf(xr[i]));
-    if (yr) m[1] = fmaxf(m[1], bf(yr[i]));
-  }
-  float s[2] = {0.f, 0.f};
-  {
-    const float nx = m[0] == -INFINITY ? 0.f : neg_scaled_max(m[0]);
-    const float ny = m[1] == -INFINITY ? 0.f : neg_scaled_max(m[1]);
-    for (int64_t i = threadIdx.x; i < a.V; i += blockDim.x) {
-      s[0] += scaled_exp2(bf(xr[i]), nx);
-      if (yr) s[1] += scaled_exp2(bf(yr[i]), ny);
+  const uint16_t* const xr = a.x + row * a.V;
+  // a teacher row out of range: row 0 is read and q is NaN below
+  const uint16_t* const yr = has_y ? a.y + max(trow, static_cast<int64_t>(0)) * a.V : nullptr;
+  const uint16_t* const kNegInf = reinterpret_cast<const uint16_t*>(&kNegInfChunk);
+  const int tid = threadIdx.x;
+  const uint32_t full = static_cast<uint32_t>(a.V / 8);  // whole chunks
+  const int tail = static_cast<int>(a.V & 7);            // logits after them: one per thread 0 .. tail - 1
+  const int64_t tail_at = full * 8LL + tid;
+  const bool in_tail = tid < tail;
+
+  // ---- pass 1: (max, sum) of the thread's chunks. The sum is relative to `ref`, a maximum of the
+  // thread's that is replaced only when a chunk exceeds it by more than kSlack: nearly every chunk
+  // then costs one compare instead of a rescaling, and exp2 of the shifted logits stays far from
+  // overflow (2^(1.44 kSlack) per element).
+  struct Running {
+    float max = -INFINITY, ref = -INFINITY, nref = 0.f, sum = 0.f;
+  } run[2];
+  uint32_t best = 0;  // the first of the thread's chunks that holds its maximum
+  constexpr float kSlack = 24.f;
+  auto absorb = [&](const uint4& v, Running& r) __attribute__((always_inline)) -> bool {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    float x[8];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[2 * k] = lo_bf(w[k]), x[2 * k + 1] = hi_bf(w[k]);
+    const float cm = max3_raw(max3_raw(x[0], x[1], x[2]), max3_raw(x[3], x[4], x[5]), max3_raw(x[6], x[7], x[7]));
+    const bool grow = cm > r.max;
+    r.max = grow ? cm : r.max;
+    if (__any(cm > r.ref + kSlack)) {
+      if (cm > r.ref) {
+        r.sum = sum_relative_to(r.ref, r.sum, cm);
+        r.ref = cm;
+        r.nref = neg_scaled_max(cm);
+      }
+    }
+    float e[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) e[k] = scaled_exp2(x[k], r.nref);
+    r.sum += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+    return grow;
+  };
+  // Steps of THREADS chunks (one per thread), two at a time, the next two loading meanwhile. A lane
+  // past the last whole chunk reads the -inf chunk, which adds nothing.
+  constexpr int kSteps = 2;
+  const int groups = static_cast<int>((full + kSteps * THREADS - 1) / (kSteps * THREADS));
+  uint4 nx[kSteps], ny[kSteps];
+  auto fetch = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      const uint32_t c = static_cast<uint32_t>(g * kSteps + u) * THREADS + tid;
+      nx[u] = load_chunk(c < full ? xr + c * 8LL : kNegInf);
+      if (has_y) ny[u] = load_chunk(c < full ? yr + c * 8LL : kNegInf);
+    }
+  };
+  if (groups > 0) fetch(0);
+  for (int g = 0; g < groups; ++g) {
+    uint4 xv[kSteps], yv[kSteps];
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      xv[u] = nx[u];
+      if (has_y) yv[u] = ny[u];
+    }
+    fetch(min(g + 1, groups - 1));  // the last group stays for pass 2, which begins with it
+#pragma unroll
+    for (int u = 0; u < kSteps; ++u) {
+      if (absorb(xv[u], run[0])) best = static_cast<uint32_t>(g * kSteps + u) * THREADS + tid;
+      if (has_y) absorb(yv[u], run[1]);
     }
   }
+  // (max, sum relative to it); a sum that is NaN, of a NaN or +inf logit, stays so
+  float m[2], s[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    m[i] = run[i].max;
+    s[i] = sum_relative_to(run[i].ref, run[i].sum, m[i]);
+  }
+  if (in_tail) {
+    const float x = bf(xr[tail_at]);
+    if (x > m[0]) best = full;
+    merge_max_sum(m[0], s[0], x, x == x ? 1.f : x);
+    if (has_y) {
+      const float y = bf(yr[tail_at]);
+      merge_max_sum(m[1], s[1], y, y == y ? 1.f : y);
+    }
+  }
+  const float own_max = m[0];
   block_max_sum<2>(m, s, scratch);
+
   if (a.amax) {  // first NaN, else first maximum (torch.argmax)
     uint32_t key = kNoKey;
-    for (int64_t i = threadIdx.x; i < a.V; i += blockDim.x)
-      key = min(key, argmax_key(bf(xr[i]), m[0], static_cast<uint32_t>(i)));
-    for (int off = 32; off > 0; off >>= 1)
-      key = min(key, static_cast<uint32_t>(__shfl_xor(static_cast<int>(key), off)));
-    __shared__ uint32_t keys[8];
-    if ((threadIdx.x & 63) == 0) keys[threadIdx.x >> 6] = key;
+    if (s[0] == s[0]) {
+      // no NaN and a finite maximum: a thread that holds it looks for it in the chunk it noted
+      if (own_max == m[0]) {
+        if (best == full) {
+          key = argmax_key(m[0], m[0], static_cast<uint32_t>(tail_at));
+        } else {
+          for (int k = 7; k >= 0; --k)
+            if (bf(xr[best * 8LL + k]) == m[0]) key = argmax_key(m[0], m[0], static_cast<uint32_t>(best * 8 + k));
+        }
+      }
+    } else {
+      for (int64_t i = tid; i < a.V; i += THREADS)
+        key = min(key, argmax_key(bf(xr[i]), m[0], static_cast<uint32_t>(i)));
+    }
+    key = wave_allmin(key);
+    if ((tid & 63) == 0) keys[tid >> 6] = key;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int w = 1; w < static_cast<int>(blockDim.x >> 6); ++w) key = min(key, keys[w]);
+    if (tid == 0) {
+      for (int w = 1; w < THREADS / 64; ++w) key = min(key, keys[w]);
       a.amax[row] = static_cast<int64_t>(key & 0x7fffffffu);
     }
   }
+
+  // ---- pass 2: the L1 masses
   const float nmx = neg_scaled_max(m[0]), nmy = neg_scaled_max(m[1]);
-  const float ix = 1.f / s[0], iy = 1.f / s[1];
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  const float ix = 1.f / s[0], iy = trow < 0 ? NAN : 1.f / s[1];
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};  // |p-q|, mass p>q, mass p<q, mass p==q
   if (has_y) {
-    for (int64_t i = threadIdx.x; i < a.V; i += blockDim.x) {
-      const float p = scaled_exp2(bf(xr[i]), nmx) * ix;
-      const float q = yr ? scaled_exp2(bf(yr[i]), nmy) * iy : NAN;
-      l1_terms(p, q, acc[0], acc[1], acc[2], acc[3]);
+    // Everything in units of 1 / S_x: p - q is (e_x - e_y S_x / S_y) / S_x, one fused multiply-add
+    // (identical rows: the ratio is 1 and the difference exactly 0). The masses above and below are
+    // summed each by itself, so a small one beside a large one keeps its digits; a chunk with an
+    // exact tie also tells ties from the rest, and so does a row with NaN probabilities on either
+    // side (every difference is NaN), whose p all counts as neither.
+    const float ratio = trow < 0 ? NAN : s[0] / s[1];
+    auto masses = [&](const uint4& xv, const uint4& yv) __attribute__((always_inline)) {
+      const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w}, yw[4] = {yv.x, yv.y, yv.z, yv.w};
+      float p[8], d[8], low = INFINITY;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t wx = xw[k >> 1], wy = yw[k >> 1];
+        p[k] = scaled_exp2((k & 1) ? hi_bf(wx) : lo_bf(wx), nmx);
+        d[k] = fmaf(-scaled_exp2((k & 1) ? hi_bf(wy) : lo_bf(wy), nmy), ratio, p[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) low = min3_abs_raw(low, d[k], d[k + 1]);
+      acc[0] += ((fabsf(d[0]) + fabsf(d[1])) + (fabsf(d[2]) + fabsf(d[3]))) +
+                ((fabsf(d[4]) + fabsf(d[5])) + (fabsf(d[6]) + fabsf(d[7])));
+      if (low > 0.f && low < INFINITY) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const bool above = d[k] > 0.f;
+          acc[1] += above ? p[k] : 0.f;
+          acc[2] += above ? 0.f : p[k];
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          acc[1] += d[k] > 0.f ? p[k] : 0.f;
+          acc[2] += d[k] < 0.f ? p[k] : 0.f;
+          acc[3] += (d[k] > 0.f) | (d[k] < 0.f) ? 0.f : p[k];
+        }
+      }
+    };
+    for (int g = groups - 1; g >= 0; --g) {
+      uint4 xv[kSteps], yv[kSteps];
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u) xv[u] = nx[u], yv[u] = ny[u];
+      fetch(max(g - 1, 0));
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u) masses(xv[u], yv[u]);
     }
+    if (in_tail) {
+      const float p = scaled_exp2(bf(xr[tail_at]), nmx), q = scaled_exp2(bf(yr[tail_at]), nmy);
+      const float d = fmaf(-q, ratio, p);
+      acc[0] += fabsf(d);
+      acc[1] += d > 0.f ? p : 0.f;
+      acc[2] += d < 0.f ? p : 0.f;
+      acc[3] += (d > 0.f) | (d < 0.f) ? 0.f : p;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] *= ix;
     block_reduce<4, false>(acc, scratch);
   }
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     const float lse = logf(s[0]) + m[0];
     float* st = a.stats + row * kStats;
     st[0] = m[0]; st[1] = ix; st[2] = m[1]; st[3] = iy;
@@ -577,28 +743,14 @@ __global__ void __launch_bounds__(256) loss_fwd_streaming(LossArgs a) {
 }
 
 // dx = g_ce * (p - onehot(t)) + g_l1 * p * centered  (tiled_l1.py:107-127 for the L1 part).
-__device__ __forceinline__ float grad_elem(float x, float y, const float* st, float gl1, float gce,
-                                           bool is_target, bool has_y) {
-  const float p = scaled_exp2(x, neg_scaled_max(st[0])) * st[1];
-  float d = 0.f;
-  if (has_y) {
-    const float q = scaled_exp2(y, neg_scaled_max(st[2])) * st[3];
-    const float pos = st[4], neg = st[5], zero = st[6];
-    const float centered = p > q ? 2.f * neg + zero : (p < q ? -2.f * pos - zero : neg - pos);
-    d = p * centered * gl1;
-  }
-  if (gce != 0.f) d += gce * (p - (is_target ? 1.f : 0.f));
-  return d;
-}
-
-// Vectorised path (V % 8 == 0): each workgroup pass covers 256 consecutive chunks of eight logits
-// of one row, so the row's statistics, upstream gradients, target and teacher index are
-// wave-uniform and read through the scalar cache; only the logits and dx use the vector memory
-// path.
+// Each workgroup pass covers 256 consecutive chunks of eight logits of one row, so the row's
+// statistics, upstream gradients, target and teacher index are wave-uniform and read through the
+// scalar cache; only the logits and dx use the vector memory path (16-byte accesses at any
+// alignment; a row's last, partial chunk goes element by element).
 constexpr int kBwdThreads = 256;
 
 __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) {
-  const int64_t per_row = a.V / 8;
+  const int64_t per_row = (a.V + 7) / 8;
   const int64_t segs_per_row = (per_row + kBwdThreads - 1) / kBwdThreads;
   const int64_t segs = a.rows * segs_per_row;
   const bool has_y = a.y != nullptr;
@@ -622,7 +774,7 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
     }
     if (chunk >= per_row) continue;
     // dx = p * (L1 weight of the element's case + g_ce) - g_ce at the target, p = e_x / S_x with
-    // e = exp2(v log2e - max log2e) (scaled_exp2, as grad_elem). Per row: the three case weights
+    // e = exp2(v log2e - max log2e) (scaled_exp2, as the forward). Per row: the three case weights
     // times 1/S_x, and r = (1/S_y) / (1/S_x), so p against q is e_x against e_y * r (identical rows:
     // r = 1 and e_x == e_y, the p == q case).
     const float nmx = neg_scaled_max(st[0]), nmy = neg_scaled_max(st[2]);
@@ -635,8 +787,9 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
     const int64_t col0 = chunk * 8;
     const uint16_t* xr = a.x + row * a.V;
     const uint16_t* yr = (has_y && trow >= 0) ? a.y + trow * a.V : nullptr;
-    const uint4 xs = *reinterpret_cast<const uint4*>(xr + col0);
-    const uint4 ys = yr ? *reinterpret_cast<const uint4*>(yr + col0) : make_uint4(0, 0, 0, 0);
+    const int live = static_cast<int>(min(a.V - col0, static_cast<int64_t>(8)));
+    const uint4 xs = live == 8 ? load_chunk(xr + col0) : load_part(xr + col0, live);
+    const uint4 ys = !yr ? make_uint4(0, 0, 0, 0) : live == 8 ? load_chunk(yr + col0) : load_part(yr + col0, live);
     const uint32_t xw[4] = {xs.x, xs.y, xs.z, xs.w};
     const uint32_t yw[4] = {ys.x, ys.y, ys.z, ys.w};
     float d[8];
@@ -651,7 +804,7 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
           const float qs = scaled_exp2(y, nmy) * r;
           k = ex > qs ? k_gt : (ex < qs ? k_lt : k_eq);
         } else {
-          k = NAN;  // teacher row out of range: NaN, as grad_elem gives
+          k = NAN;  // teacher row out of range
         }
       }
       d[e] = ex * k;
@@ -665,55 +818,13 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
     uint32_t out[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[e] = pack_bf16x2(d[2 * e], d[2 * e + 1]);
-    *reinterpret_cast<uint4*>(a.dx + row * a.V + col0) = make_uint4(out[0], out[1], out[2], out[3]);
-  }
-}
-
-template <bool VEC>
-__global__ void __launch_bounds__(256) loss_bwd_kernel(LossArgs a) {
-  const int64_t per_row = VEC ? a.V / 8 : a.V;
-  const int64_t total = a.rows * per_row;
-  const bool has_y = a.y != nullptr;
-  for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t row = t / per_row;
-    const int64_t col0 = (t - row * per_row) * (VEC ? 8 : 1);
-    float st[kStats];
-#pragma unroll
-    for (int i = 0; i < kStats; ++i) st[i] = a.stats[row * kStats + i];
-    const float gl1 = (has_y && a.g_l1) ? a.g_l1[row] : 0.f;
-    float gce = 0.f;
-    int64_t tgt = -1;
-    if (a.g_ce) {
-      tgt = a.target[row];
-      gce = tgt == a.ignore_index ? 0.f : a.g_ce[row];
-    }
-    int64_t trow = 0;
-    if (has_y) {
-      trow = a.yidx ? a.yidx[row] : row;
-      if (trow < 0 || trow >= a.trows) trow = -1;
-    }
-    const uint16_t* xr = a.x + row * a.V;
-    const uint16_t* yr = (has_y && trow >= 0) ? a.y + trow * a.V : nullptr;
-    if (VEC) {
-      const uint4 xs = *reinterpret_cast<const uint4*>(xr + col0);
-      const uint4 ys = yr ? *reinterpret_cast<const uint4*>(yr + col0) : make_uint4(0, 0, 0, 0);
-      const uint32_t xw[4] = {xs.x, xs.y, xs.z, xs.w};
-      const uint32_t yw[4] = {ys.x, ys.y, ys.z, ys.w};
-      uint32_t out[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float y0 = yr ? __uint_as_float(yw[e] << 16) : NAN;
-        const float y1 = yr ? __uint_as_float(yw[e] & 0xffff0000u) : NAN;
-        const float d0 = grad_elem(__uint_as_float(xw[e] << 16), y0, st, gl1, gce, col0 + 2 * e == tgt, has_y);
-        const float d1 = grad_elem(__uint_as_float(xw[e] & 0xffff0000u), y1, st, gl1, gce, col0 + 2 * e + 1 == tgt, has_y);
-        out[e] = pack_bf16x2(d0, d1);
-      }
-      *reinterpret_cast<uint4*>(a.dx + row * a.V + col0) = make_uint4(out[0], out[1], out[2], out[3]);
+    uint16_t* const dr = a.dx + row * a.V + col0;
+    if (live == 8) {
+      store_chunk(dr, make_uint4(out[0], out[1], out[2], out[3]));
     } else {
-      const float y = yr ? bf(yr[col0]) : NAN;
-      const float d = grad_elem(bf(xr[col0]), y, st, gl1, gce, col0 == tgt, has_y);
-      a.dx[row * a.V + col0] = f32_to_bf16_bits(d);
+#pragma unroll
+      for (int e = 0; e < 7; ++e)
+        if (e < live) dr[e] = static_cast<uint16_t>(out[e >> 1] >> ((e & 1) * 16));
     }
   }
 }
@@ -732,6 +843,12 @@ void launch_walk(const LossArgs& a, dim3 walk, dim3 block, hipStream_t s) {
     if (a.amax) hipLaunchKernelGGL((loss_fwd_persistent<NV, true, false>), walk, block, 0, s, a);
     else hipLaunchKernelGGL((loss_fwd_persistent<NV, false, false>), walk, block, 0, s, a);
   }
+}
+
+template <int THREADS>
+void launch_streaming(const LossArgs& a, dim3 grid, hipStream_t s) {
+  if (a.y) hipLaunchKernelGGL((loss_fwd_streaming<THREADS, true>), grid, dim3(THREADS), 0, s, a);
+  else hipLaunchKernelGGL((loss_fwd_streaming<THREADS, false>), grid, dim3(THREADS), 0, s, a);
 }
 
 int launch_fwd(const LossArgs& a, hipStream_t s) {
@@ -753,25 +870,18 @@ int launch_fwd(const LossArgs& a, hipStream_t s) {
     launch_walk<4>(a, walk, block, s);
   } else if (vec && a.V <= kWalkThreads * 8 * 8) {
     launch_walk<8>(a, walk, block, s);
+  } else if (a.V <= 8192) {  // one workgroup per row, as many threads as its chunks keep busy
+    launch_streaming<256>(a, grid, s);
   } else {
-    hipLaunchKernelGGL(loss_fwd_streaming, grid, dim3(256), 0, s, a);
+    launch_streaming<512>(a, grid, s);
   }
   return check_launch("loss forward");
 }
 
 int launch_bwd(const LossArgs& a, hipStream_t s) {
-  const bool vec = a.V % 8 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 &&
-                   (!a.y || (reinterpret_cast<uintptr_t>(a.y) & 15) == 0) &&
-                   (reinterpret_cast<uintptr_t>(a.dx) & 15) == 0;
-  const int64_t work = a.rows * (vec ? a.V / 8 : a.V);
-  const int64_t blocks = std::min<int64_t>((work + 255) / 256, 256 * 64);
-  if (vec) {
-    const int64_t segs = a.rows * ((a.V / 8 + kBwdThreads - 1) / kBwdThreads);
-    const int64_t grid = std::min<int64_t>(segs, 256 * 64);
-    hipLaunchKernelGGL(loss_bwd_rows_kernel, dim3(static_cast<uint32_t>(grid)), dim3(kBwdThreads), 0, s, a);
-  } else {
-    hipLaunchKernelGGL(loss_bwd_kernel<false>, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s, a);
-  }
+  const int64_t segs = a.rows * (((a.V + 7) / 8 + kBwdThreads - 1) / kBwdThreads);
+  const int64_t grid = std::min<int64_t>(segs, 256 * 64);
+  hipLaunchKernelGGL(loss_bwd_rows_kernel, dim3(static_cast<uint32_t>(grid)), dim3(kBwdThreads), 0, s, a);
   return check_launch("loss backward");
 }
 

@@ -1,0 +1,60 @@
+"""The two-pass loss forward and the backward at any vocabulary and row alignment (V % 8 != 0, rows
+past the row walk's reach), against the fp64 oracle at the edges of their chunks and steps: fewer
+logits than a chunk, a lone tail, exact multiples of a step (8 x 256 or 512 logits) and one more or
+less, and the 256- to 512-thread border. Bars as in tests/test_gpu_loss.py; the argmax exact."""
+
+import numpy as np
+import pytest
+import torch
+
+from aspec_amd.loss import ce_l1_from_logits, cross_entropy
+from oracle import loss as L
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("vocab", [1, 7, 9, 2047, 2049, 4095, 4097, 8191, 8193, 16383, 32769, 40960, 65537, 152063])
+def test_any_vocabulary(gpu, vocab):
+    rows, trows = 5, 3
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    x = (torch.randn(rows, vocab, device=gpu, generator=g) * 3).to(torch.bfloat16)
+    y = (torch.randn(trows, vocab, device=gpu, generator=g) * 3).to(torch.bfloat16)
+    x[0] += (torch.arange(vocab, device=gpu) * (60.0 / vocab)).to(torch.bfloat16)  # a rising maximum
+    x[1] = y[2]                                                                       # identical rows
+    x[2, vocab // 2:] = x[2].max()                                                    # tied maxima
+    index = torch.tensor([0, 2, 1, 1, 0], device=gpu)
+    t = torch.tensor([vocab - 1, 0, vocab // 2, -100, vocab // 3], device=gpu)
+    gce, gl1 = torch.randn(rows, device=gpu, generator=g), torch.randn(rows, device=gpu, generator=g)
+    xin = x.clone().requires_grad_()
+    ce, l1, amax = ce_l1_from_logits(xin, t, y, teacher_indices=index, return_argmax=True)
+    ((ce * gce).sum() + (l1 * gl1).sum()).backward()
+    xd, yd, td = x.double().cpu().numpy(), y[index].double().cpu().numpy(), t.cpu().numpy()
+    np.testing.assert_allclose(ce.detach().double().cpu().numpy(), L.cross_entropy(xd, td), atol=2e-5, rtol=2e-6)
+    np.testing.assert_allclose(l1.detach().double().cpu().numpy(), L.l1(xd, yd), atol=2e-6, rtol=2e-6)
+    assert l1[1].item() == 0.0
+    assert torch.equal(amax.cpu(), torch.as_tensor(np.argmax(xd, axis=-1)))  # the first maximum
+    ref = torch.as_tensor(L.cross_entropy_grad(xd, td, gce.double().cpu().numpy())
+                          + L.l1_grad(xd, yd, gl1.double().cpu().numpy()))
+    assert (xin.grad.double().cpu() - ref).norm() <= 0.01 * ref.norm() + 1e-6
+    torch.testing.assert_close(xin.grad.cpu(), ref.to(torch.bfloat16), atol=1e-6, rtol=0.02)
+    torch.testing.assert_close(cross_entropy(x, t), ce.detach(), atol=0, rtol=0)
+
+
+def test_rows_off_alignment(gpu):
+    """A 2-byte-aligned view of a vocabulary that is a multiple of eight: the same numbers as the
+    aligned copy (which the row walk serves) within its rounding."""
+    rows, vocab = 4, 4096
+    g = torch.Generator(device=gpu).manual_seed(5)
+    flat = torch.randn(1 + rows * vocab, device=gpu, generator=g).to(torch.bfloat16)
+    off = flat[1:].view(rows, vocab)
+    y = torch.randn(rows, vocab, device=gpu, generator=g).to(torch.bfloat16)
+    t = torch.randint(0, vocab, (rows,), device=gpu, generator=g)
+    grads = []
+    for x in (off, off.clone()):
+        xin = x.detach().requires_grad_()
+        ce, l1 = ce_l1_from_logits(xin, t, y)
+        grads.append((ce.detach(), l1.detach(), torch.autograd.grad(ce.sum() + l1.sum(), xin)[0]))
+    assert off.data_ptr() % 16 == 2
+    torch.testing.assert_close(grads[0][0], grads[1][0], atol=2e-5, rtol=2e-6)
+    torch.testing.assert_close(grads[0][1], grads[1][1], atol=2e-6, rtol=2e-6)
+    torch.testing.assert_close(grads[0][2], grads[1][2], atol=1e-6, rtol=0.02)
