@@ -2,7 +2,7 @@
 // and backward, alone or fused. HBM-bound streaming reductions.
 //
 // Forward:
-//   row walk (V % 8 == 0, V <= 512*8*8): one 512-thread workgroup per CU walks the rows; each row
+//   row walk (V % 8 == 0, V <= 512*8*8): one or two 512-thread workgroups per CU walk the rows; each row
 //   of draft and teacher logits is read from HBM exactly once into registers while the previous
 //   row is reduced (max / sum / |p - q| / sign masses);
 //   streaming path (any V, any alignment): one workgroup per row, two passes over the row in
@@ -164,6 +164,11 @@ constexpr int kWalkThreads = 512;  // threads of the persistent row walk (8 wave
 // Eight bf16 -inf: what the row walk's lanes past the end of a row load.
 __device__ const uint4 kNegInfChunk = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
 constexpr int kWalkWaves = kWalkThreads / 64;
+// Workgroups of the walk per CU. A row of up to 16384 tokens leaves half the registers free, and a
+// second workgroup works while the first waits at a row's barriers: 8192 rows x 8192 tokens 110 ->
+// 93 us, x 16000 149 -> 134 us, with dlogits x 8192 160 -> 126 us (a third workgroup spills). With
+// dlogits at 16384 tokens two spill already (214 against 210 us).
+constexpr int walk_groups(int nv, bool grad) { return nv >= 8 || (nv == 4 && grad) ? 1 : 2; }
 
 // Per-thread max and exp2 values of NV chunks of eight bf16 logits (chunk j of thread t holds
 // row elements (j * kWalkThreads + t) * 8 .. +7; value i of `e` is element i % 8 of chunk i / 8).
@@ -303,7 +308,8 @@ __device__ __forceinline__ void block_sums(float (&v)[NP], uint32_t& key, float*
 // dx = p * (L1 case weight * g_l1 + g_ce) - g_ce at the target (the backward's formula), into `dx`
 // (which may be the logits themselves: the row has been read by then).
 template <int NV, bool ARGMAX, bool HAS_Y, bool GRAD = false>
-__global__ void __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(kWalkThreads)
+__attribute__((amdgpu_waves_per_eu(2 * walk_groups(NV, GRAD), 2 * walk_groups(NV, GRAD))))
 loss_fwd_persistent(LossArgs args) {
   static_assert(!GRAD || HAS_Y, "the fused gradient needs a teacher");
   __shared__ float merge_slots[4 * kWalkWaves];  // (max, sum) of x and y per wave
@@ -830,7 +836,9 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
 }
 
 template <int NV>
-void launch_walk(const LossArgs& a, dim3 walk, dim3 block, hipStream_t s) {
+void launch_walk(const LossArgs& a, int cus, hipStream_t s) {
+  const dim3 block(kWalkThreads);
+  const dim3 walk(static_cast<uint32_t>(std::min<int64_t>(a.rows, cus * walk_groups(NV, a.dx != nullptr))));
   if (a.dx) {  // the fused forward + dlogits (teacher present, checked by the entry point)
     if (a.amax) hipLaunchKernelGGL((loss_fwd_persistent<NV, true, true, true>), walk, block, 0, s, a);
     else hipLaunchKernelGGL((loss_fwd_persistent<NV, false, true, true>), walk, block, 0, s, a);
@@ -859,17 +867,15 @@ int launch_fwd(const LossArgs& a, hipStream_t s) {
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     return set_error(ASPEC_ERR_RUNTIME, "cannot query the GPU's compute-unit count");
-  const dim3 walk(static_cast<uint32_t>(std::min<int64_t>(a.rows, cus)));
-  const dim3 block(kWalkThreads);
   if (a.dx && !(vec && a.V <= kWalkThreads * 8 * 8 && (reinterpret_cast<uintptr_t>(a.dx) & 15) == 0))
     return set_error(ASPEC_ERR_UNSUPPORTED, "the fused loss forward + dlogits needs V %% 8 == 0, V <= %d "
                      "and 16-byte aligned rows", kWalkThreads * 8 * 8);
   if (vec && a.V <= kWalkThreads * 8 * 2) {
-    launch_walk<2>(a, walk, block, s);
+    launch_walk<2>(a, cus, s);
   } else if (vec && a.V <= kWalkThreads * 8 * 4) {
-    launch_walk<4>(a, walk, block, s);
+    launch_walk<4>(a, cus, s);
   } else if (vec && a.V <= kWalkThreads * 8 * 8) {
-    launch_walk<8>(a, walk, block, s);
+    launch_walk<8>(a, cus, s);
   } else if (a.V <= 8192) {  // one workgroup per row, as many threads as its chunks keep busy
     launch_streaming<256>(a, grid, s);
   } else {
