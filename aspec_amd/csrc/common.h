@@ -28,6 +28,17 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t v) {
   return __uint_as_float(static_cast<uint32_t>(v) << 16);
 }
 
+// Eight consecutive 16-bit elements as one 16-byte global access at any 2-byte alignment (the
+// target serves unaligned global accesses; odd row lengths put rows there).
+typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t ChunkWords;
+__device__ __forceinline__ uint4 load_chunk(const uint16_t* p) {
+  const u32x4 v = *(const __attribute__((address_space(1))) ChunkWords*)(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void store_chunk(uint16_t* p, const uint4& v) {
+  *(__attribute__((address_space(1))) ChunkWords*)(p) = u32x4{v.x, v.y, v.z, v.w};
+}
+
 // Round-to-nearest-even float -> bf16 bits (NaN stays NaN), hardware conversion.
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
   const __attribute__((ext_vector_type(2))) float x = {f, 0.f};

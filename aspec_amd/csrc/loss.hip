@@ -139,16 +139,7 @@ __device__ __forceinline__ void block_max_sum(float (&m)[NP], float (&s)[NP], fl
 __device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
-// Eight consecutive bf16 as one 16-byte access at any 2-byte alignment, and the first n of them
-// element by element (the rest 0).
-typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t ChunkWords;
-__device__ __forceinline__ uint4 load_chunk(const uint16_t* p) {
-  const u32x4 v = *(const __attribute__((address_space(1))) ChunkWords*)(p);
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ void store_chunk(uint16_t* p, const uint4& v) {
-  *(__attribute__((address_space(1))) ChunkWords*)(p) = u32x4{v.x, v.y, v.z, v.w};
-}
+// The first n of eight consecutive bf16, element by element (the rest 0).
 __device__ __forceinline__ uint4 load_part(const uint16_t* p, int n) {
   uint32_t w[4];
 #pragma unroll

@@ -10,14 +10,21 @@
 //
 // One 512-thread workgroup owns a row; the row lives in registers as packed bf16 (NV chunks of
 // eight per thread, up to 98304 tokens; longer rows are read again from global memory on each
-// pass) and nothing is sorted. scaled is a non-decreasing function of the bf16 value,
-// so the top-p boundary is the smallest 16-bit bf16 key whose strictly-greater mass is <= top_p:
-// a binary search of 16 block reductions over the key space (top-k: the same over counts). One
-// pass then forms the boundary's tie group in scaled values (a temperature can merge neighbouring
-// bf16 values into one fp32 value), the kept count within it follows from the group's mass per
-// token, and, when the group is cut, a search over token indices finds the last kept token. A
-// token is kept iff its scaled key is above the boundary key, or equal and its index <= last.
-// Masses are fp32 per token, summed in fp64 in a fixed order (deterministic).
+// pass) and nothing is sorted. A row takes three passes: the maximum; the total mass, with every
+// token's mass and count added to a histogram of LDS bins, 1/32 nat of scaled logit each; and, the
+// bin that holds the boundary found by a scan, the exact mass above that bin and the list of its
+// tokens. One wave then finishes on the list: the boundary key (a binary search over the bin's few
+// distinct bf16 values), its tie group in scaled values (a temperature can merge neighbouring bf16
+// values into one fp32 value), the kept count within the group from its mass per token, and, when
+// the group is cut, the index of the last kept token. A token is kept iff its scaled value is above
+// the boundary's, or equal and its index <= last.
+//
+// The histogram's masses (fp32, any order) only propose a bin: it is taken when the exact mass above
+// it is <= top_p of the total and the mass with it is not, else its neighbour is tried. Masses are
+// fp32 per token, summed in fp64: over the row in a fixed order, and over a bin's list exactly (its
+// masses lie within e^(1/32) of each other, so at most 2048 of them sum without rounding). So the
+// result does not depend on the order of the atomics. A boundary in the last, open bin or in one of
+// more than 2048 tokens (all-equal rows) is found by binary searches over the whole row instead.
 #include <cmath>
 
 #include "common.h"
@@ -28,6 +35,9 @@ namespace {
 constexpr int kSampThreads = 512;
 constexpr int kSampWaves = kSampThreads / 64;
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kBins = 2048;        // bins of 1/32 nat below the maximum: 64 nats, the last one open
+constexpr float kBinsPerNat = 32.f;
+constexpr int kListCap = 2048;     // tokens of the boundary's bin that the list holds
 constexpr uint32_t kNegInfBits = 0xff80u;  // bf16 -inf: the padding of a row's tail
 
 // per-row, per-side record (8 words); the sampled-L1 row holds draft, teacher, then the masses
@@ -97,18 +107,31 @@ __device__ __forceinline__ float e_of(float x, const RowCtx& c) {
 }
 __device__ __forceinline__ float ord_of(float x, const RowCtx& c) { return c.temp ? u_of(x, c) : x; }
 
+// the value of an ordered key
+__device__ __forceinline__ float value_of_key(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+
 __device__ __forceinline__ RowCtx ctx_of(const SideStats& s) {
   return RowCtx{s.m, s.rcp_t, (s.flags & kFlagTemp) != 0};
 }
+// A row's support as the passes test it: kept iff the sort value is above `bound`, or equal (-0
+// equals +0) at an index <= last. A row without a filter has bound -inf and every index.
+struct Support {
+  float bound;
+  int32_t last;
+};
+__device__ __forceinline__ Support support_of(const SideStats& s) {
+  return (s.flags & kFlagAll) ? Support{-INFINITY, 0x7fffffff} : Support{value_of_key(s.okey), s.last};
+}
 // branch-free: evaluated for every token of a pass
-__device__ __forceinline__ bool kept(const SideStats& s, uint32_t okey, int64_t idx) {
-  return ((s.flags & kFlagAll) != 0) | (okey > s.okey) | ((okey == s.okey) & (idx <= s.last));
+__device__ __forceinline__ bool kept(const Support& s, float ord, int32_t idx) {
+  return (ord > s.bound) | ((ord == s.bound) & (idx <= s.last));
 }
 // probability of a token after filtering (0 outside the support)
-__device__ __forceinline__ float prob(const SideStats& s, uint32_t h, int64_t idx) {
-  const RowCtx c = ctx_of(s);
+__device__ __forceinline__ float prob(const Support& s, const RowCtx& c, float zinv, uint32_t h, int32_t idx) {
   const float x = bf16f(h);
-  return kept(s, ord_key(ord_of(x, c)), idx) ? e_of(x, c) * s.zinv : 0.0f;
+  return kept(s, ord_of(x, c), idx) ? e_of(x, c) * zinv : 0.0f;
 }
 
 // ---- block reductions over the 8 waves, fixed order, every thread gets the total ---------------
@@ -116,20 +139,36 @@ struct Red {
   double slot[2][kSampWaves];
 };
 
+__device__ __forceinline__ double join_d(uint32_t lo, uint32_t hi) {
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  return join_d(dpp_u32<CTRL>(static_cast<uint32_t>(b)), dpp_u32<CTRL>(static_cast<uint32_t>(b >> 32)));
+}
+// wave_allsum (common.h) for doubles: every lane gets the sum, added in a fixed pairing
 __device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  v += dpp_d<0x141>(v);
+  v += dpp_d<0x140>(v);
+  uint64_t b = __builtin_bit_cast(uint64_t, v);
+  uint32_t lo = static_cast<uint32_t>(b), hi = static_cast<uint32_t>(b >> 32);
+  auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  v = join_d(l[0], h[0]) + join_d(l[1], h[1]);
+  b = __builtin_bit_cast(uint64_t, v);
+  lo = static_cast<uint32_t>(b), hi = static_cast<uint32_t>(b >> 32);
+  l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return join_d(l[0], h[0]) + join_d(l[1], h[1]);
 }
 __device__ __forceinline__ uint32_t wave_sum_u(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_allreduce_bits(v, [](uint32_t a, uint32_t b) { return a + b; });
 }
-__device__ __forceinline__ float wave_max_f(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
+  return wave_allreduce_bits(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 // A value every lane holds alike, moved to scalar registers (the row's statistics and search
 // bounds then take no vector registers beside the row itself).
@@ -141,17 +180,14 @@ __device__ __forceinline__ double uniform(double v) {
 }
 
 // Two slot sets used alternately: the barrier of the call in between separates the reads of one
-// call from the writes of the call after next. Lane l of every 8-lane group reads wave l's slot
-// and a butterfly over the group adds them (a fixed pairing: every lane gets the same total).
+// call from the writes of the call after next. Every thread adds the eight waves' slots in one
+// fixed pairing.
 __device__ __forceinline__ double block_total(double wave_value, Red& r, int& ph) {
   double* slot = r.slot[ph];
   ph ^= 1;
   if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = wave_value;
   __syncthreads();
-  double s = slot[threadIdx.x & (kSampWaves - 1)];
-#pragma unroll
-  for (int o = kSampWaves / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kSampWaves);
-  return uniform(s);
+  return uniform(((slot[0] + slot[1]) + (slot[2] + slot[3])) + ((slot[4] + slot[5]) + (slot[6] + slot[7])));
 }
 __device__ __forceinline__ double block_sum(double v, Red& r, int& ph) {
   return block_total(wave_sum_d(v), r, ph);
@@ -159,22 +195,30 @@ __device__ __forceinline__ double block_sum(double v, Red& r, int& ph) {
 __device__ __forceinline__ int64_t block_count(uint32_t v, Red& r, int& ph) {
   return static_cast<int64_t>(block_total(static_cast<double>(wave_sum_u(v)), r, ph));
 }
-__device__ __forceinline__ float block_max(float v, Red& r, int& ph) {
+// the row maximum, and whether any thread's `bad` is set
+__device__ __forceinline__ float block_max(float v, bool bad, bool& any_bad, Red& r, int& ph) {
   double* slot = r.slot[ph];
   ph ^= 1;
-  v = wave_max_f(v);
-  if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = static_cast<double>(v);
+  v = wave_allmax(v);
+  // a NaN slot marks a wave with a bad token
+  const double mine = __any(bad) ? __builtin_nan("") : static_cast<double>(v);
+  if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = mine;
   __syncthreads();
-  double s = slot[threadIdx.x & (kSampWaves - 1)];
+  double m = slot[0];
+  any_bad = m != m;
 #pragma unroll
-  for (int o = kSampWaves / 2; o > 0; o >>= 1) s = fmax(s, __shfl_xor(s, o, kSampWaves));
-  return static_cast<float>(uniform(s));
+  for (int w = 1; w < kSampWaves; ++w) {
+    const double o = slot[w];
+    any_bad |= o != o;
+    m = fmax(m, o);
+  }
+  return static_cast<float>(uniform(m));
 }
 
 // ---- rows -------------------------------------------------------------------------------------
 // Chunk c of thread t is tokens (c * 512 + t) * 8 .. + 7; tokens past V read as bf16 -inf.
-__device__ __forceinline__ uint4 load_chunk(const uint16_t* row, int64_t V, bool vec, int64_t base) {
-  if (vec && base < V) return *reinterpret_cast<const uint4*>(row + base);
+__device__ __forceinline__ uint4 row_chunk(const uint16_t* row, int64_t V, int64_t base) {
+  if (base + 8 <= V) return load_chunk(row + base);
   uint32_t w[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -200,13 +244,11 @@ __device__ __forceinline__ uint32_t half_of(const uint32_t (&w)[4], int j) {
 // indices) is recomputed in that pass instead of being hoisted out of the searches' loops.
 template <int NV>
 struct RegRow {
-  static constexpr bool kCacheable = NV <= 8;  // exp values kept too, up to 32768 tokens
-  static constexpr int kSlots = NV * 8;
   uint4 r[NV];
-  __device__ __forceinline__ void load(const uint16_t* row, int64_t V, bool vec) {
+  __device__ __forceinline__ void load(const uint16_t* row, int64_t V) {
 #pragma unroll
     for (int c = 0; c < NV; ++c)
-      r[c] = load_chunk(row, V, vec, (static_cast<int64_t>(c) * kSampThreads + threadIdx.x) * 8);
+      r[c] = row_chunk(row, V, (static_cast<int64_t>(c) * kSampThreads + threadIdx.x) * 8);
   }
   template <typename G>
   __device__ __forceinline__ void chunks(G&& g) {
@@ -223,14 +265,11 @@ struct RegRow {
 // A row read again from global memory on every pass, for vocabularies beyond the registers' reach
 // (the row stays in the caches between a workgroup's passes).
 struct GlobalRow {
-  static constexpr bool kCacheable = false;
-  static constexpr int kSlots = 1;
   const uint16_t* p;
   int64_t V;
-  bool vec;
   int n;
-  __device__ __forceinline__ void load(const uint16_t* row, int64_t V_, bool vec_) {
-    p = row, V = V_, vec = vec_;
+  __device__ __forceinline__ void load(const uint16_t* row, int64_t V_) {
+    p = row, V = V_;
     n = static_cast<int>((V + 8LL * kSampThreads - 1) / (8LL * kSampThreads));
   }
   template <typename G>
@@ -238,7 +277,7 @@ struct GlobalRow {
     const int32_t t8 = static_cast<int32_t>(threadIdx.x) * 8;
     for (int c = 0; c < n; ++c) {
       const int32_t base = c * kSampThreads * 8 + t8;
-      const uint4 v = load_chunk(p, V, vec, base);
+      const uint4 v = row_chunk(p, V, base);
       const uint32_t w[4] = {v.x, v.y, v.z, v.w};
       g(0, base, w);
     }
@@ -257,64 +296,173 @@ __device__ __forceinline__ void fence(T&... v) {
   (fence1(v), ...);
 }
 
-// f(slot, bf16 bits, token index) over the thread's tokens, in a fixed order; end() after each
-// chunk (fences the pass's accumulators)
+// f(bf16 bits, token index) over the thread's tokens, in a fixed order; end() after each chunk
+// (fences the pass's accumulators)
 template <typename Row, typename F, typename G>
 __device__ __forceinline__ void for_each(Row& row, F&& f, G&& end) {
   row.chunks([&](int c, int32_t base, const uint32_t (&w)[4]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      f(c * 8 + 2 * k, w[k] & 0xffffu, base + 2 * k);
-      f(c * 8 + 2 * k + 1, w[k] >> 16, base + 2 * k + 1);
+      f(w[k] & 0xffffu, base + 2 * k);
+      f(w[k] >> 16, base + 2 * k + 1);
     }
     end();
   });
 }
 
-// One side's support and normaliser. Rows with a NaN or no finite maximum get kFlagNaN (the
-// reference's softmax gives NaN there).
-template <typename Row>
-__device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const SideParams P, Red& red,
-                                                     int& ph) {
-  constexpr bool kCache = Row::kCacheable;
-  SideStats st = {};
-  float mx = -INFINITY;
-  uint32_t bad = 0;
-  for_each(r, [&](int, uint32_t h, int64_t) {
-    bad |= (h & 0x7fffu) > 0x7f80u ? 1u : 0u;
-    mx = fmaxf(mx, bf16f(h));
-  }, [&] { fence(mx, bad); });
-  const float m = block_max(mx, red, ph);
-  const bool nan_row = block_count(bad, red, ph) > 0 || !(m > -INFINITY && m < INFINITY);
-  st.m = m;
-  st.rcp_t = P.temp ? P.rcp_t : 1.0f;
-  st.flags = P.temp ? kFlagTemp : 0u;
-  if (nan_row) {
-    st.flags |= kFlagNaN;
-    return st;
-  }
-  const RowCtx cx{m, st.rcp_t, P.temp != 0};
-  float ec[kCache ? Row::kSlots : 1];
-  if constexpr (kCache) for_each(r, [&](int s, uint32_t h, int64_t) { ec[s] = e_of(bf16f(h), cx); }, [] {});
-  auto E = [&](int s, uint32_t h) -> float {
-    if constexpr (kCache) return ec[s];
-    else return e_of(bf16f(h), cx);
-  };
+// LDS of one row's support search.
+struct Work {
+  Red red;
+  float mass[kBins];
+  uint32_t count[kBins];
+  uint32_t key[kListCap];  // the list: x_key and index of the tokens of the bin looked at
+  int32_t idx[kListCap];
+  float wave_mass[kSampWaves];
+  uint32_t wave_count[kSampWaves];
+  uint32_t n;        // tokens appended to the list
+  int32_t bin_p, bin_k;
+  int32_t verdict;   // what the list's wave found: see Verdict
+  uint32_t okey;
+  int32_t last;
+  double z;
+};
+enum Verdict { kFound, kHigher, kLower };
 
-  // top-p boundary (okey_p, n_p of c_p ties kept)
+// The distance of a sort value below the maximum in bins, as a float: its integer part is the bin
+// (the last bin takes everything beyond). A function of the scaled value, so tokens that tie share
+// a bin.
+__device__ __forceinline__ float bin_of(float u) { return fminf(-u * kBinsPerNat, static_cast<float>(kBins - 1)); }
+
+// The end of the search on one bin's list, by one wave: `above` is the exact mass and `before` the
+// count of the tokens in higher bins, lim = top_p times the row's mass; use_k says whether top_k's
+// boundary lies in this bin.
+__device__ __forceinline__ void search_list(Work& w, int n, const RowCtx& cx, bool use_p, double lim, double above,
+                                            bool use_k, int64_t top_k, int64_t before) {
+  const int lane = threadIdx.x & 63;
+  auto value = [&](int i) { return bf16f(x_bits_of_key(w.key[i])); };
+  auto okey_at = [&](int i) { return ord_key(ord_of(value(i), cx)); };
+  uint32_t kmin = 0xffffu, kmax = 0;
+  double mass = 0.0;
+  for (int i = lane; i < n; i += kWave) {
+    kmin = min(kmin, w.key[i]);
+    kmax = max(kmax, w.key[i]);
+    mass += e_of(value(i), cx);
+  }
+  kmin = wave_allmin(kmin);
+  kmax = wave_max_u(kmax);
+  mass = wave_sum_d(mass);
+  bool have_p = false;
+  if (use_p) {
+    if (above > lim) {  // the top-p boundary lies in a higher bin
+      if (lane == 0) w.verdict = kHigher;
+      return;
+    }
+    have_p = above + mass > lim;
+    if (!have_p && !use_k) {
+      if (lane == 0) w.verdict = kLower;
+      return;
+    }
+  }
+  uint32_t okey = 0;
+  int64_t keep = 0, ties = 0;
+  // (sort key, kept ties, ties) of a boundary at x_key k: `room(mass, count)` gives the kept ties
+  // from the mass and count of the list's tokens above it
+  auto boundary = [&](uint32_t k, auto&& room) {
+    const uint32_t o = ord_key(ord_of(bf16f(x_bits_of_key(k)), cx));
+    double m = 0.0;
+    uint32_t over = 0, same = 0;
+    for (int i = lane; i < n; i += kWave) {
+      const uint32_t oi = okey_at(i);
+      if (oi > o) m += e_of(value(i), cx);
+      over += oi > o ? 1u : 0u;
+      same += oi == o ? 1u : 0u;
+    }
+    const int64_t c = wave_sum_u(same);
+    const int64_t left = room(wave_sum_d(m), static_cast<int64_t>(wave_sum_u(over)), c,
+                              e_of(bf16f(x_bits_of_key(k)), cx));
+    // both filters keep a prefix of the order: the shorter one wins
+    if (ties == 0 || o > okey || (o == okey && left < keep)) okey = o, keep = left, ties = c;
+  };
+  if (have_p) {
+    uint32_t lo = kmin, hi = kmax;  // the smallest key with a strictly greater mass <= lim
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      double f = 0.0;
+      for (int i = lane; i < n; i += kWave) f += w.key[i] > mid ? e_of(value(i), cx) : 0.0f;
+      if (above + wave_sum_d(f) <= lim) hi = mid;
+      else lo = mid + 1;
+    }
+    boundary(lo, [&](double m, int64_t, int64_t c, float eb) -> int64_t {
+      // the j-th tie (0-based, index order) has mass above + m + j * eb before it
+      if (!(eb > 0.0f)) return c;
+      const double q = floor((lim - (above + m)) / static_cast<double>(eb));
+      return q + 1.0 >= static_cast<double>(c) ? c : static_cast<int64_t>(q) + 1;
+    });
+  }
+  if (use_k) {
+    uint32_t lo = kmin, hi = kmax;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      uint32_t c = 0;
+      for (int i = lane; i < n; i += kWave) c += w.key[i] > mid ? 1u : 0u;
+      if (before + wave_sum_u(c) <= top_k - 1) hi = mid;
+      else lo = mid + 1;
+    }
+    boundary(lo, [&](double, int64_t over, int64_t, float) -> int64_t { return top_k - before - over; });
+  }
+  // the index of the last kept tie: the smallest j with `keep` ties at indices <= j
+  int32_t last = 0x7fffffff;
+  if (keep < ties) {
+    int32_t lo = 0x7fffffff, hi = 0;
+    for (int i = lane; i < n; i += kWave) {
+      lo = min(lo, w.idx[i]);
+      hi = max(hi, w.idx[i]);
+    }
+    lo = static_cast<int32_t>(wave_allmin(static_cast<uint32_t>(lo)));
+    hi = static_cast<int32_t>(wave_max_u(static_cast<uint32_t>(hi)));
+    while (lo < hi) {
+      const int32_t mid = (lo + hi) >> 1;
+      uint32_t c = 0;
+      for (int i = lane; i < n; i += kWave) c += ((w.idx[i] <= mid) & (okey_at(i) == okey)) ? 1u : 0u;
+      if (static_cast<int64_t>(wave_sum_u(c)) >= keep) hi = mid;
+      else lo = mid + 1;
+    }
+    last = lo;
+  }
+  // the kept mass: the bins above, the list's tokens above the boundary, the kept ties
+  double m = 0.0;
+  float eb = 0.0f;
+  for (int i = lane; i < n; i += kWave) {
+    const uint32_t oi = okey_at(i);
+    const float e = e_of(value(i), cx);
+    if (oi > okey) m += e;
+    if (oi == okey) eb = e;
+  }
+  m = wave_sum_d(m);
+  eb = wave_allmax(eb);
+  if (lane == 0) {
+    w.verdict = kFound;
+    w.okey = okey;
+    w.last = last;
+    w.z = above + m + static_cast<double>(eb) * static_cast<double>(keep);
+  }
+}
+
+// The support by binary searches over the whole row (16-bit keys, then token indices): for a
+// boundary that the list cannot hold. `total` is the row's mass.
+template <typename Row>
+__device__ __forceinline__ void search_row(Row& r, int64_t V, const SideParams& P, const RowCtx& cx, double total,
+                                        SideStats& st, Red& red, int& ph) {
   bool have_p = false, have_k = false;
   uint32_t okey_p = 0, okey_k = 0;
   int64_t n_p = 0, c_p = 0, n_k = 0, c_k = 0;
   if (P.use_p) {
-    double se = 0.0;
-    for_each(r, [&](int s, uint32_t h, int64_t) { se += E(s, h); }, [&] { fence(se); });
-    const double lim = static_cast<double>(P.top_p) * block_sum(se, red, ph);
+    const double lim = static_cast<double>(P.top_p) * total;
     uint32_t lo = 0, hi = 0xffffu;
     while (lo < hi) {
       const uint32_t mid = (lo + hi) >> 1;
       double f = 0.0;
-      for_each(r, [&](int s, uint32_t h, int64_t) { f += x_key(h) > mid ? E(s, h) : 0.0f; },
-               [&] { fence(f); });
+      for_each(r, [&](uint32_t h, int32_t) { f += x_key(h) > mid ? e_of(bf16f(h), cx) : 0.0f; }, [&] { fence(f); });
       if (block_sum(f, red, ph) <= lim) hi = mid;
       else lo = mid + 1;
     }
@@ -325,9 +473,9 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
       const float eb = e_of(xb, cx);
       double f = 0.0;
       uint32_t c = 0;
-      for_each(r, [&](int s, uint32_t h, int64_t) {
+      for_each(r, [&](uint32_t h, int32_t) {
         const uint32_t k = ord_key(ord_of(bf16f(h), cx));
-        f += k > okey_p ? E(s, h) : 0.0f;
+        f += k > okey_p ? e_of(bf16f(h), cx) : 0.0f;
         c += k == okey_p ? 1u : 0u;
       }, [&] { fence(f, c); });
       const double above = block_sum(f, red, ph);
@@ -347,14 +495,13 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     while (lo < hi) {
       const uint32_t mid = (lo + hi) >> 1;
       uint32_t cnt = 0;
-      for_each(r, [&](int, uint32_t h, int64_t) { cnt += x_key(h) > mid ? 1u : 0u; },
-               [&] { fence(cnt); });
+      for_each(r, [&](uint32_t h, int32_t) { cnt += x_key(h) > mid ? 1u : 0u; }, [&] { fence(cnt); });
       if (block_count(cnt, red, ph) <= P.top_k - 1) hi = mid;
       else lo = mid + 1;
     }
     okey_k = ord_key(ord_of(bf16f(x_bits_of_key(lo)), cx));
     uint32_t a = 0, c = 0;
-    for_each(r, [&](int, uint32_t h, int64_t) {
+    for_each(r, [&](uint32_t h, int32_t) {
       const uint32_t k = ord_key(ord_of(bf16f(h), cx));
       a += k > okey_k ? 1u : 0u;
       c += k == okey_k ? 1u : 0u;
@@ -383,7 +530,7 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     while (lo < hi) {
       const int64_t mid = (lo + hi) >> 1;
       uint32_t c = 0;
-      for_each(r, [&](int, uint32_t h, int64_t idx) {
+      for_each(r, [&](uint32_t h, int32_t idx) {
         c += ((idx <= mid) & (ord_key(ord_of(bf16f(h), cx)) == okey)) ? 1u : 0u;
       }, [&] { fence(c); });
       if (block_count(c, red, ph) >= n) hi = mid;
@@ -392,14 +539,143 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     st.last = static_cast<int32_t>(lo);
   }
   double z = 0.0;
-  uint32_t nm = 0;
-  for_each(r, [&](int s, uint32_t h, int64_t idx) {
+  const Support sup = support_of(st);
+  for_each(r, [&](uint32_t h, int32_t idx) {
     const float x = bf16f(h);
-    z += kept(st, ord_key(ord_of(x, cx)), idx) ? E(s, h) : 0.0f;
-    nm += x == m ? 1u : 0u;
-  }, [&] { fence(z, nm); });
+    z += kept(sup, ord_of(x, cx), idx) ? e_of(x, cx) : 0.0f;
+  }, [&] { fence(z); });
   st.zinv = static_cast<float>(1.0 / block_sum(z, red, ph));
-  st.nmax = static_cast<int32_t>(block_count(nm, red, ph));
+}
+
+// One side's support and normaliser. Rows with a NaN or no finite maximum get kFlagNaN (the
+// reference's softmax gives NaN there).
+template <typename Row>
+__device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const SideParams P, Work& w, int& ph) {
+  const int tid = threadIdx.x;
+  SideStats st = {};
+  float mx = -INFINITY;
+  uint32_t mag = 0;  // the largest magnitude bits: above 0x7f80 is a NaN
+  for_each(r, [&](uint32_t h, int32_t) {
+    mag = max(mag, h & 0x7fffu);
+    mx = fmaxf(mx, bf16f(h));
+  }, [&] { fence(mx, mag); });
+  bool has_nan;
+  const float m = block_max(mx, mag > 0x7f80u, has_nan, w.red, ph);
+  st.m = m;
+  st.rcp_t = P.temp ? P.rcp_t : 1.0f;
+  st.flags = P.temp ? kFlagTemp : 0u;
+  if (has_nan || !(m > -INFINITY && m < INFINITY)) {
+    st.flags |= kFlagNaN;
+    return st;
+  }
+  const RowCtx cx{m, st.rcp_t, P.temp != 0};
+  const bool filter = P.use_p || P.use_k;
+  if (filter) {
+    for (int i = tid; i < kBins; i += kSampThreads) w.mass[i] = 0.0f, w.count[i] = 0u;
+    if (tid == 0) w.n = 0, w.bin_p = kBins - 1, w.bin_k = kBins - 1;
+    __syncthreads();
+  }
+  // the total mass, the tokens equal to the maximum and the histogram
+  double se = 0.0;
+  uint32_t nm = 0;
+  for_each(r, [&](uint32_t h, int32_t) {
+    const float x = bf16f(h);
+    const float u = u_of(x, cx);
+    const float e = e_of(x, cx);
+    se += e;
+    nm += x == m ? 1u : 0u;
+    if (filter) {
+      const int b = static_cast<int>(bin_of(u));
+      if (b < kBins - 1) {
+        if (P.use_p) __hip_atomic_fetch_add(&w.mass[b], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (P.use_k) __hip_atomic_fetch_add(&w.count[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+  }, [&] { fence(se, nm); });
+  const double total = block_sum(se, w.red, ph);  // its barrier also completes the histogram
+  st.nmax = static_cast<int32_t>(block_count(nm, w.red, ph));
+  if (!filter) {
+    st.flags |= kFlagAll;
+    st.last = 0x7fffffff;
+    st.zinv = static_cast<float>(1.0 / total);
+    return st;
+  }
+  // The bins that hold the top-p and top-k boundaries: thread t scans bins 4t .. 4t+3.
+  const double lim = static_cast<double>(P.top_p) * total;
+  constexpr int kPer = kBins / kSampThreads;
+  float own_m[kPer];
+  uint32_t own_c[kPer];
+  float sum_m = 0.0f;
+  uint32_t sum_c = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    own_m[i] = w.mass[tid * kPer + i];
+    own_c[i] = w.count[tid * kPer + i];
+    sum_m += own_m[i];
+    sum_c += own_c[i];
+  }
+  float inc_m = sum_m;
+  uint32_t inc_c = sum_c;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const float fm = __shfl_up(inc_m, o);
+    const uint32_t fc = __shfl_up(inc_c, o);
+    if ((tid & 63) >= o) inc_m += fm, inc_c += fc;
+  }
+  if ((tid & 63) == 63) w.wave_mass[tid >> 6] = inc_m, w.wave_count[tid >> 6] = inc_c;
+  __syncthreads();
+  float run_m = inc_m - sum_m;
+  uint32_t run_c = inc_c - sum_c;
+  for (int i = 0; i < (tid >> 6); ++i) run_m += w.wave_mass[i], run_c += w.wave_count[i];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    run_m += own_m[i];
+    if (P.use_p && static_cast<double>(run_m) > lim) atomicMin(&w.bin_p, tid * kPer + i);
+    if (P.use_k) {
+      const uint32_t next = run_c + own_c[i];
+      if (static_cast<int64_t>(next) >= P.top_k) atomicMin(&w.bin_k, tid * kPer + i);
+      w.count[tid * kPer + i] = run_c;  // now the count of the tokens in higher bins
+      run_c = next;
+    }
+  }
+  __syncthreads();
+  const int bin_k = P.use_k ? w.bin_k : kBins;
+  int bin = P.use_p ? min(w.bin_p, bin_k) : bin_k;
+  while (true) {
+    if (bin >= kBins - 1) break;
+    const float lo = static_cast<float>(bin), hi = static_cast<float>(bin + 1);
+    double f = 0.0;
+    for_each(r, [&](uint32_t h, int32_t idx) {
+      const float x = bf16f(h);
+      const float b = bin_of(u_of(x, cx));
+      f += b < lo ? e_of(x, cx) : 0.0f;
+      if (b >= lo && b < hi) {
+        const uint32_t at = __hip_atomic_fetch_add(&w.n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (at < kListCap) w.key[at] = x_key(h), w.idx[at] = idx;
+      }
+    }, [&] { fence(f); });
+    const double above = block_sum(f, w.red, ph);  // its barrier also completes the list
+    const uint32_t n = w.n;
+    if (n > kListCap) break;
+    if (tid < kWave)
+      search_list(w, static_cast<int>(n), cx, P.use_p, lim, above, bin == bin_k, P.top_k,
+                  P.use_k ? static_cast<int64_t>(w.count[bin]) : 0);
+    __syncthreads();
+    const int verdict = w.verdict;
+    if (verdict == kFound) {
+      st.okey = w.okey;
+      st.last = w.last;
+      st.zinv = static_cast<float>(1.0 / w.z);
+      __syncthreads();  // w is reused by the row's other side
+      return st;
+    }
+    bin += verdict == kHigher ? -1 : 1;
+    if (bin < 0) break;
+    __syncthreads();
+    if (tid == 0) w.n = 0;
+    __syncthreads();
+  }
+  search_row(r, V, P, cx, total, st, w.red, ph);
   return st;
 }
 
@@ -426,21 +702,18 @@ __device__ __forceinline__ SideStats load_side(const float* src) {
   return s;
 }
 
-__device__ __forceinline__ bool row_vec(const uint16_t* p, int64_t V) {
-  return V % 8 == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
-}
-
 // ---- sampling_logits: the filtered fp32 logits and their gradient ------------------------------
 template <typename Row>
 __global__ void __launch_bounds__(kSampThreads) sampling_fwd_kernel(SampledArgs a) {
-  __shared__ Red red;
+  __shared__ Work work;
   int ph = 0;
   const int64_t row = blockIdx.x, V = a.V;
   const SideParams px = a.px;
   Row r;
-  r.load(a.x + row * V, V, row_vec(a.x, V));
-  const SideStats s = compute_support(r, V, px, red, ph);
+  r.load(a.x + row * V, V);
+  const SideStats s = compute_support(r, V, px, work, ph);
   const RowCtx cx = ctx_of(s);
+  const Support sup = support_of(s);
   float* out = a.out + row * V;
   const bool nan_row = (s.flags & kFlagNaN) != 0;
   const bool vec_out = V % 4 == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
@@ -450,7 +723,7 @@ __global__ void __launch_bounds__(kSampThreads) sampling_fwd_kernel(SampledArgs 
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float v = ord_of(bf16f(half_of(w, j)), cx);
-      o[j] = nan_row ? __builtin_nanf("") : (kept(s, ord_key(v), base + j) ? v : -INFINITY);
+      o[j] = nan_row ? __builtin_nanf("") : (kept(sup, v, base + j) ? v : -INFINITY);
     }
     if (vec_out && base + 8 <= V) {
       *reinterpret_cast<float4*>(out + base) = make_float4(o[0], o[1], o[2], o[3]);
@@ -471,9 +744,10 @@ __global__ void __launch_bounds__(kSampThreads) sampling_bwd_kernel(SampledArgs 
   int ph = 0;
   const int64_t row = blockIdx.x, V = a.V;
   Row r;
-  r.load(a.x + row * V, V, row_vec(a.x, V));
+  r.load(a.x + row * V, V);
   const SideStats s = load_side(a.stats + row * kSideWords);
   const RowCtx cx = ctx_of(s);
+  const Support sup = support_of(s);
   const float* g = a.gout + row * V;
   uint16_t* dx = a.dx + row * V;
   const bool nan_row = (s.flags & kFlagNaN) != 0;
@@ -500,7 +774,7 @@ __global__ void __launch_bounds__(kSampThreads) sampling_bwd_kernel(SampledArgs 
       grads(base, gv);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        sg += kept(s, ord_key(ord_of(bf16f(half_of(w, j)), cx)), base + j) ? gv[j] : 0.0f;
+        sg += kept(sup, ord_of(bf16f(half_of(w, j)), cx), base + j) ? gv[j] : 0.0f;
       fence(sg);
     });
     share = static_cast<float>(block_sum(sg, red, ph) * static_cast<double>(s.rcp_t) / s.nmax);
@@ -516,7 +790,7 @@ __global__ void __launch_bounds__(kSampThreads) sampling_bwd_kernel(SampledArgs 
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const float x = bf16f(half_of(w, 2 * k + h));
-        float v = kept(s, ord_key(ord_of(x, cx)), base + 2 * k + h) ? gv[2 * k + h] * s.rcp_t : 0.0f;
+        float v = kept(sup, ord_of(x, cx), base + 2 * k + h) ? gv[2 * k + h] * s.rcp_t : 0.0f;
         v -= x == s.m ? share : 0.0f;
         d[h] = nan_row ? __builtin_nanf("") : v;
       }
@@ -534,7 +808,7 @@ __global__ void __launch_bounds__(kSampThreads) sampling_bwd_kernel(SampledArgs 
 // ---- sampled L1 ---------------------------------------------------------------------------------
 template <typename Row>
 __global__ void __launch_bounds__(kSampThreads) sampled_l1_fwd_kernel(SampledArgs a) {
-  __shared__ Red red;
+  __shared__ Work work;
   int ph = 0;
   const int64_t row = blockIdx.x;
   int64_t yrow = row;
@@ -556,21 +830,22 @@ __global__ void __launch_bounds__(kSampThreads) sampled_l1_fwd_kernel(SampledArg
   const uint16_t* xr = a.x + row * V;
   const uint16_t* yr = a.y + yrow * V;
   Row r;
-  r.load(yr, V, row_vec(a.y, V));
-  const SideStats sy = compute_support(r, V, py, red, ph);
-  r.load(xr, V, row_vec(a.x, V));
-  const SideStats sx = compute_support(r, V, px, red, ph);
+  r.load(yr, V);
+  const SideStats sy = compute_support(r, V, py, work, ph);
+  r.load(xr, V);
+  const SideStats sx = compute_support(r, V, px, work, ph);
   const bool nan_row = ((sx.flags | sy.flags) & kFlagNaN) != 0;
   double l1 = 0.0, pos = 0.0, neg = 0.0, zero = 0.0;
   if (!nan_row) {
-    const bool yvec = row_vec(a.y, V);
+    const RowCtx cx = ctx_of(sx), cy = ctx_of(sy);
+    const Support kx = support_of(sx), ky = support_of(sy);
     r.chunks([&](int, int32_t base, const uint32_t (&wx)[4]) {
-      const uint4 yc = load_chunk(yr, V, yvec, base);
+      const uint4 yc = row_chunk(yr, V, base);
       const uint32_t wy[4] = {yc.x, yc.y, yc.z, yc.w};
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float p = prob(sx, half_of(wx, j), base + j);
-        const float q = prob(sy, half_of(wy, j), base + j);
+        const float p = prob(kx, cx, sx.zinv, half_of(wx, j), base + j);
+        const float q = prob(ky, cy, sy.zinv, half_of(wy, j), base + j);
         l1 += fabsf(p - q);
         pos += p > q ? p : 0.0f;
         neg += p < q ? p : 0.0f;
@@ -579,10 +854,10 @@ __global__ void __launch_bounds__(kSampThreads) sampled_l1_fwd_kernel(SampledArg
       fence(l1, pos, neg, zero);
     });
   }
-  const double t_l1 = block_sum(l1, red, ph);
-  const double t_pos = block_sum(pos, red, ph);
-  const double t_neg = block_sum(neg, red, ph);
-  const double t_zero = block_sum(zero, red, ph);
+  const double t_l1 = block_sum(l1, work.red, ph);
+  const double t_pos = block_sum(pos, work.red, ph);
+  const double t_neg = block_sum(neg, work.red, ph);
+  const double t_zero = block_sum(zero, work.red, ph);
   if (threadIdx.x == 0) {
     float* st = a.stats + row * kL1Words;
     store_side(st, sx);
@@ -598,15 +873,17 @@ __global__ void __launch_bounds__(kSampThreads) sampled_l1_fwd_kernel(SampledArg
 // d logits = g / T_draft * p * (sign(p - q) - sum p sign(p - q)), written per case without
 // cancellation: 2 neg + zero (p > q), -(2 pos + zero) (p < q), neg - pos (p == q), where pos, neg
 // and zero are the draft mass on tokens with p > q, p < q and p == q. Each workgroup takes one
-// 2048-token segment of a row per loop step.
+// 2048-token segment of a row per loop step, eight tokens per thread in 16-byte accesses.
 __global__ void __launch_bounds__(256) sampled_l1_bwd_kernel(SampledArgs a) {
   const int64_t segs = (a.V + 2047) / 2048;
   for (int64_t unit = blockIdx.x; unit < a.rows * segs; unit += gridDim.x) {
     const int64_t row = unit / segs;
-    const int64_t base = (unit - row * segs) * 2048 + static_cast<int64_t>(threadIdx.x) * 8;
+    const int32_t base = static_cast<int32_t>(unit - row * segs) * 2048 + static_cast<int32_t>(threadIdx.x) * 8;
     const float* st = a.stats + row * kL1Words;
     const SideStats sx = load_side(st);
     const SideStats sy = load_side(st + kSideWords);
+    const RowCtx cx = ctx_of(sx), cy = ctx_of(sy);
+    const Support kx = support_of(sx), ky = support_of(sy);
     const float pos = st[16], neg = st[17], zero = st[18];
     const float g = a.g_l1[row] * sx.rcp_t;
     const bool nan_row = ((sx.flags | sy.flags) & kFlagNaN) != 0;
@@ -615,17 +892,27 @@ __global__ void __launch_bounds__(256) sampled_l1_bwd_kernel(SampledArgs a) {
       yrow = a.yidx[row];
       if (yrow < 0 || yrow >= a.trows) yrow = 0;  // NaN row (flagged by the forward)
     }
-    const uint16_t* xr = a.x + row * a.V;
-    const uint16_t* yr = a.y + yrow * a.V;
-    uint16_t* dr = a.dx + row * a.V;
     if (base >= a.V) continue;
+    const uint4 xc = row_chunk(a.x + row * a.V, a.V, base);
+    const uint4 yc = row_chunk(a.y + yrow * a.V, a.V, base);
+    const uint32_t wx[4] = {xc.x, xc.y, xc.z, xc.w}, wy[4] = {yc.x, yc.y, yc.z, yc.w};
     const float w_gt = g * (2.0f * neg + zero), w_lt = -g * (2.0f * pos + zero), w_eq = g * (neg - pos);
-    for (int j = 0; j < 8 && base + j < a.V; ++j) {
-      const int64_t idx = base + j;
-      const float p = prob(sx, xr[idx], idx);
-      const float q = prob(sy, yr[idx], idx);
-      const float d = p * (p > q ? w_gt : (p < q ? w_lt : w_eq));
-      dr[idx] = f32_to_bf16_bits(nan_row ? __builtin_nanf("") : d);
+    float d[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float p = prob(kx, cx, sx.zinv, half_of(wx, j), base + j);
+      const float q = prob(ky, cy, sy.zinv, half_of(wy, j), base + j);
+      d[j] = nan_row ? __builtin_nanf("") : p * (p > q ? w_gt : (p < q ? w_lt : w_eq));
+    }
+    const uint32_t out[4] = {pack_bf16x2(d[0], d[1]), pack_bf16x2(d[2], d[3]), pack_bf16x2(d[4], d[5]),
+                             pack_bf16x2(d[6], d[7])};
+    uint16_t* dr = a.dx + row * a.V + base;
+    if (base + 8 <= a.V) {
+      store_chunk(dr, make_uint4(out[0], out[1], out[2], out[3]));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 7; ++j)
+        if (base + j < a.V) dr[j] = static_cast<uint16_t>(half_of(out, j));
     }
   }
 }
