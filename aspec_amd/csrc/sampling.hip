@@ -244,8 +244,10 @@ __device__ __forceinline__ uint32_t half_of(const uint32_t (&w)[4], int j) {
 // indices) is recomputed in that pass instead of being hoisted out of the searches' loops.
 template <int NV>
 struct RegRow {
+  const uint16_t* p;
   uint4 r[NV];
   __device__ __forceinline__ void load(const uint16_t* row, int64_t V) {
+    p = row;
 #pragma unroll
     for (int c = 0; c < NV; ++c)
       r[c] = row_chunk(row, V, (static_cast<int64_t>(c) * kSampThreads + threadIdx.x) * 8);
@@ -313,8 +315,8 @@ __device__ __forceinline__ void for_each(Row& row, F&& f, G&& end) {
 // LDS of one row's support search.
 struct Work {
   Red red;
-  float mass[kBins];
-  uint32_t count[kBins];
+  float mass[kBins + kWave];  // past kBins: where the last bin's adds go, a word per lane, never read
+  uint32_t count[kBins + kWave];
   uint32_t key[kListCap];  // the list: x_key and index of the tokens of the bin looked at
   int32_t idx[kListCap];
   float wave_mass[kSampWaves];
@@ -449,9 +451,9 @@ __device__ __forceinline__ void search_list(Work& w, int n, const RowCtx& cx, bo
 }
 
 // The support by binary searches over the whole row (16-bit keys, then token indices): for a
-// boundary that the list cannot hold. `total` is the row's mass.
-template <typename Row>
-__device__ __forceinline__ void search_row(Row& r, int64_t V, const SideParams& P, const RowCtx& cx, double total,
+// boundary that the list cannot hold, read from the caches in rolled loops (unrolled over a row's
+// registers, this rare path was most of the file's code). `total` is the row's mass.
+__device__ __forceinline__ void search_row(GlobalRow& r, int64_t V, const SideParams& P, const RowCtx& cx, double total,
                                         SideStats& st, Red& red, int& ph) {
   bool have_p = false, have_k = false;
   uint32_t okey_p = 0, okey_k = 0;
@@ -578,20 +580,32 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
   // the total mass, the tokens equal to the maximum and the histogram
   double se = 0.0;
   uint32_t nm = 0;
-  for_each(r, [&](uint32_t h, int32_t) {
-    const float x = bf16f(h);
-    const float u = u_of(x, cx);
-    const float e = e_of(x, cx);
-    se += e;
-    nm += x == m ? 1u : 0u;
-    if (filter) {
-      const int b = static_cast<int>(bin_of(u));
-      if (b < kBins - 1) {
-        if (P.use_p) __hip_atomic_fetch_add(&w.mass[b], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (P.use_k) __hip_atomic_fetch_add(&w.count[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
+  // (one branch per filter and chunk, none per token)
+  const int sink = kBins + (tid & 63);
+  r.chunks([&](int, int32_t base, const uint32_t (&v)[4]) {
+    float e[8];
+    int at[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float x = bf16f(half_of(v, j));
+      e[j] = e_of(x, cx);
+      se += e[j];
+      nm += x == m ? 1u : 0u;
+      const int b = static_cast<int>(bin_of(u_of(x, cx)));
+      at[j] = b < kBins - 1 ? b : sink;
     }
-  }, [&] { fence(se, nm); });
+    if (P.use_p && base < V) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        __hip_atomic_fetch_add(&w.mass[at[j]], e[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (P.use_k && base < V) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        __hip_atomic_fetch_add(&w.count[at[j]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    fence(se, nm);
+  });
   const double total = block_sum(se, w.red, ph);  // its barrier also completes the histogram
   st.nmax = static_cast<int32_t>(block_count(nm, w.red, ph));
   if (!filter) {
@@ -645,15 +659,24 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     if (bin >= kBins - 1) break;
     const float lo = static_cast<float>(bin), hi = static_cast<float>(bin + 1);
     double f = 0.0;
-    for_each(r, [&](uint32_t h, int32_t idx) {
-      const float x = bf16f(h);
-      const float b = bin_of(u_of(x, cx));
-      f += b < lo ? e_of(x, cx) : 0.0f;
-      if (b >= lo && b < hi) {
-        const uint32_t at = __hip_atomic_fetch_add(&w.n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (at < kListCap) w.key[at] = x_key(h), w.idx[at] = idx;
+    r.chunks([&](int, int32_t base, const uint32_t (&v)[4]) {
+      uint32_t in_bin = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x = bf16f(half_of(v, j));
+        const float b = bin_of(u_of(x, cx));
+        f += b < lo ? e_of(x, cx) : 0.0f;
+        in_bin |= ((b >= lo) & (b < hi)) ? 1u << j : 0u;
       }
-    }, [&] { fence(f); });
+      for (; in_bin; in_bin &= in_bin - 1) {  // few tokens of a row
+        const int j = __ffs(in_bin) - 1;
+        const uint32_t word = (j & 4) ? ((j & 2) ? v[3] : v[2]) : ((j & 2) ? v[1] : v[0]);
+        const uint32_t h = (j & 1) ? word >> 16 : word & 0xffffu;
+        const uint32_t at = __hip_atomic_fetch_add(&w.n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (at < kListCap) w.key[at] = x_key(h), w.idx[at] = base + j;
+      }
+      fence(f);
+    });
     const double above = block_sum(f, w.red, ph);  // its barrier also completes the list
     const uint32_t n = w.n;
     if (n > kListCap) break;
@@ -675,7 +698,9 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     if (tid == 0) w.n = 0;
     __syncthreads();
   }
-  search_row(r, V, P, cx, total, st, w.red, ph);
+  GlobalRow again;
+  again.load(r.p, V);
+  search_row(again, V, P, cx, total, st, w.red, ph);
   return st;
 }
 

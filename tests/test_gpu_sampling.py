@@ -89,6 +89,27 @@ def test_tie_groups_exact(gpu, vocab):
         assert kept[:, :n].all() and not kept[:, n:].any()
 
 
+@pytest.mark.parametrize("vocab", [4097, 32000, 70001, 151936])
+@pytest.mark.parametrize("ties", [2047, 2048, 2049])
+def test_boundary_bin_edges(gpu, vocab, ties):
+    """The boundary in a bin of as many tokens as the list holds, one fewer and one more, and in the
+    open last bin (more than 64 below the maximum; top-k past the finite tokens ends among -inf).
+    Filters by count only, or with the boundary's margin far above rounding: exact."""
+    x = torch.full((2, vocab), -100.0, device=gpu)
+    x[:, 3::2][:, :ties] = 1.0  # one bin: `ties` equal tokens, below three larger ones
+    x[:, :3] = 3.0
+    x[1, 5::7] = -torch.inf
+    x = x.to(torch.bfloat16)
+    for sampling in ((1.0, 1.0, 500), (0.7, 1.0, 2000), (1.0, 1.0, ties + 1000), (1.0, 1.0, vocab - 5)):
+        want = torch.from_numpy(S.sampling_logits(_np(x), sampling).astype(np.float32))
+        assert torch.equal(sampling_logits(x, sampling).cpu(), want), sampling
+    # top-p inside the tie group: (top_p * total - above) / mass per tie, plus one
+    n3, n1 = (int((x[0] == v).sum()) for v in (3.0, 1.0))
+    e = float(np.exp(-2.0))
+    keep = n3 + int(np.floor((0.5 * (n3 + n1 * e) - n3) / e)) + 1
+    assert int(torch.isfinite(sampling_logits(x[:1], (1.0, 0.5, -1))).sum()) == keep
+
+
 @pytest.mark.parametrize("vocab", [4097, 32000, 151936])
 def test_sampling_logits_gradient(gpu, vocab):
     x = _rows(gpu, 5, vocab, 3).requires_grad_()
