@@ -625,12 +625,14 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
     s[i] = sum_relative_to(run[i].ref, run[i].sum, m[i]);
   }
   if (in_tail) {
+    // a lone logit's sum relative to itself: 1, and what merge_max_sum wants of -inf (0) and NaN
+    auto lone = [](float v) { return v == -INFINITY ? 0.f : v == v ? 1.f : v; };
     const float x = bf(xr[tail_at]);
     if (x > m[0]) best = full;
-    merge_max_sum(m[0], s[0], x, x == x ? 1.f : x);
+    merge_max_sum(m[0], s[0], x, lone(x));
     if (has_y) {
       const float y = bf(yr[tail_at]);
-      merge_max_sum(m[1], s[1], y, y == y ? 1.f : y);
+      merge_max_sum(m[1], s[1], y, lone(y));
     }
   }
   const float own_max = m[0];

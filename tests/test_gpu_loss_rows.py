@@ -58,3 +58,38 @@ def test_rows_off_alignment(gpu):
     torch.testing.assert_close(grads[0][0], grads[1][0], atol=2e-5, rtol=2e-6)
     torch.testing.assert_close(grads[0][1], grads[1][1], atol=2e-6, rtol=2e-6)
     torch.testing.assert_close(grads[0][2], grads[1][2], atol=1e-6, rtol=0.02)
+
+
+def _check_against_torch(x, y, t):
+    """CE, L1, their gradient and the argmax of the kernels against the fp64 softmax on the CPU, NaN
+    for NaN. Bars as above."""
+    g = torch.Generator().manual_seed(17)
+    w = torch.rand(2, x.shape[0], generator=g)
+    xin = x.clone().requires_grad_()
+    ce, l1, amax = ce_l1_from_logits(xin, t, y, return_argmax=True)
+    (grad,) = torch.autograd.grad((ce, l1), xin, tuple(w.to(x.device)))
+    ref = x.double().cpu().requires_grad_()
+    ref_ce = torch.nn.functional.cross_entropy(ref, t.cpu(), reduction="none")
+    ref_l1 = (ref.softmax(-1) - y.double().cpu().softmax(-1)).abs().sum(-1)
+    (ref_grad,) = torch.autograd.grad((ref_ce, ref_l1), ref, tuple(w.double()))
+    torch.testing.assert_close(ce.detach().double().cpu(), ref_ce.detach(), atol=2e-5, rtol=2e-6, equal_nan=True)
+    torch.testing.assert_close(l1.detach().double().cpu(), ref_l1.detach(), atol=2e-6, rtol=2e-6, equal_nan=True)
+    assert torch.equal(amax.cpu(), ref.detach().argmax(-1))
+    torch.testing.assert_close(grad.double().cpu(), ref_grad, atol=1e-6, rtol=0.02, equal_nan=True)
+
+
+@pytest.mark.parametrize("value", [-float("inf"), float("inf"), float("nan")])
+@pytest.mark.parametrize("vocab", [2, 7, 9, 2047, 4103, 8193, 16383, 32769, 152063])
+def test_nonfinite_tail(gpu, vocab, value):
+    """Logits that are not finite among a row's last V % 8, in the draft, the teacher and both; at
+    V < 8 that is the whole row but its first."""
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    x, y = (torch.randn(6, vocab, device=gpu, generator=g) * 3 for _ in range(2))
+    tail = min(vocab % 8, vocab - 1)
+    x[0, -1] = y[1, -1] = value
+    x[2, -tail:] = y[2, -tail:] = value
+    x[3, -tail:] = value
+    y[4, -1] = value
+    x[4, -tail] = value
+    t = torch.zeros(6, dtype=torch.long, device=gpu)
+    _check_against_torch(x.to(torch.bfloat16), y.to(torch.bfloat16), t)
