@@ -92,9 +92,14 @@ __device__ __forceinline__ float scalar_read_bf16(const uint16_t* p) {
   return __uint_as_float((a & 2) ? (w & 0xffff0000u) : (w << 16));
 }
 
-// log2-domain exponent of a logit against its row maximum: p = exp2(v*log2e - max*log2e) / sum.
-// The forward and backward kernels evaluate it with this one formula, so they classify p against
-// q identically, and identical draft/teacher rows give bitwise equal probabilities.
+// log2-domain exponent of a logit against its row maximum: p = exp2(v*log2e - max*log2e) * (1/sum).
+// Forward and backward evaluate e and the product e * (1/sum) alike and compare these two rounded
+// values, p against q, so a token that the forward counts in one of the three masses gets that
+// case's weight in the backward. For a token that holds nearly all of p and of q the two differ by
+// rounding only, and the weight of another case would be off by as much as twice its probability.
+// (The row walk forms p from its thread's maximum: the same bits wherever that is the row's, which
+// is where a row's largest tokens are.) Identical draft/teacher rows give bitwise equal
+// probabilities.
 __device__ __forceinline__ float neg_scaled_max(float m) { return -(m * kLog2e); }
 __device__ __forceinline__ float scaled_exp2(float v, float nm) { return fexp2(fmaf(v, kLog2e, nm)); }
 
@@ -668,20 +673,17 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
   const float ix = 1.f / s[0], iy = trow < 0 ? NAN : 1.f / s[1];
   float acc[4] = {0.f, 0.f, 0.f, 0.f};  // |p-q|, mass p>q, mass p<q, mass p==q
   if (has_y) {
-    // Everything in units of 1 / S_x: p - q is (e_x - e_y S_x / S_y) / S_x, one fused multiply-add
-    // (identical rows: the ratio is 1 and the difference exactly 0). The masses above and below are
-    // summed each by itself, so a small one beside a large one keeps its digits; a chunk with an
-    // exact tie also tells ties from the rest, and so does a row with NaN probabilities on either
-    // side (every difference is NaN), whose p all counts as neither.
-    const float ratio = trow < 0 ? NAN : s[0] / s[1];
+    // The masses above and below are summed each by itself, so a small one beside a large one keeps
+    // its digits; a chunk with an exact tie also tells ties from the rest, and so does a row with NaN
+    // probabilities on either side (every difference is NaN), whose p all counts as neither.
     auto masses = [&](const uint4& xv, const uint4& yv) __attribute__((always_inline)) {
       const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w}, yw[4] = {yv.x, yv.y, yv.z, yv.w};
       float p[8], d[8], low = INFINITY;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const uint32_t wx = xw[k >> 1], wy = yw[k >> 1];
-        p[k] = scaled_exp2((k & 1) ? hi_bf(wx) : lo_bf(wx), nmx);
-        d[k] = fmaf(-scaled_exp2((k & 1) ? hi_bf(wy) : lo_bf(wy), nmy), ratio, p[k]);
+        p[k] = scaled_exp2((k & 1) ? hi_bf(wx) : lo_bf(wx), nmx) * ix;
+        d[k] = p[k] - scaled_exp2((k & 1) ? hi_bf(wy) : lo_bf(wy), nmy) * iy;
       }
 #pragma unroll
       for (int k = 0; k < 8; k += 2) low = min3_abs_raw(low, d[k], d[k + 1]);
@@ -712,15 +714,13 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
       for (int u = 0; u < kSteps; ++u) masses(xv[u], yv[u]);
     }
     if (in_tail) {
-      const float p = scaled_exp2(bf(xr[tail_at]), nmx), q = scaled_exp2(bf(yr[tail_at]), nmy);
-      const float d = fmaf(-q, ratio, p);
+      const float p = scaled_exp2(bf(xr[tail_at]), nmx) * ix;
+      const float d = p - scaled_exp2(bf(yr[tail_at]), nmy) * iy;
       acc[0] += fabsf(d);
       acc[1] += d > 0.f ? p : 0.f;
       acc[2] += d < 0.f ? p : 0.f;
       acc[3] += (d > 0.f) | (d < 0.f) ? 0.f : p;
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] *= ix;
     block_reduce<4, false>(acc, scratch);
   }
   if (tid == 0) {
@@ -772,17 +772,13 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
       if (trow < 0 || trow >= a.trows) trow = -1;
     }
     if (chunk >= per_row) continue;
-    // dx = p * (L1 weight of the element's case + g_ce) - g_ce at the target, p = e_x / S_x with
-    // e = exp2(v log2e - max log2e) (scaled_exp2, as the forward). Per row: the three case weights
-    // times 1/S_x, and r = (1/S_y) / (1/S_x), so p against q is e_x against e_y * r (identical rows:
-    // r = 1 and e_x == e_y, the p == q case).
+    // dx = p * (L1 weight of the element's case + g_ce) - g_ce at the target, p = e_x * (1/S_x) with
+    // e = exp2(v log2e - max log2e) (scaled_exp2) as in the forward.
     const float nmx = neg_scaled_max(st[0]), nmy = neg_scaled_max(st[2]);
     const float pos = st[4], neg = st[5], zero = st[6];
-    const float k_gt = st[1] * ((2.f * neg + zero) * gl1 + gce);
-    const float k_lt = st[1] * ((-2.f * pos - zero) * gl1 + gce);
-    const float k_eq = st[1] * ((neg - pos) * gl1 + gce);
-    const float k_ce = st[1] * gce;  // no teacher: the CE part alone
-    const float r = st[3] / st[1];
+    const float k_gt = (2.f * neg + zero) * gl1 + gce;
+    const float k_lt = (-2.f * pos - zero) * gl1 + gce;
+    const float k_eq = (neg - pos) * gl1 + gce;
     const int64_t col0 = chunk * 8;
     const uint16_t* xr = a.x + row * a.V;
     const uint16_t* yr = (has_y && trow >= 0) ? a.y + trow * a.V : nullptr;
@@ -795,18 +791,18 @@ __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) 
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float x = (e & 1) ? __uint_as_float(xw[e >> 1] & 0xffff0000u) : __uint_as_float(xw[e >> 1] << 16);
-      const float ex = scaled_exp2(x, nmx);
-      float k = k_ce;
+      const float p = scaled_exp2(x, nmx) * st[1];
+      float k = gce;  // no teacher: the CE part alone
       if (has_y) {
         if (yr) {
           const float y = (e & 1) ? __uint_as_float(yw[e >> 1] & 0xffff0000u) : __uint_as_float(yw[e >> 1] << 16);
-          const float qs = scaled_exp2(y, nmy) * r;
-          k = ex > qs ? k_gt : (ex < qs ? k_lt : k_eq);
+          const float q = scaled_exp2(y, nmy) * st[3];
+          k = p > q ? k_gt : (p < q ? k_lt : k_eq);
         } else {
           k = NAN;  // teacher row out of range
         }
       }
-      d[e] = ex * k;
+      d[e] = p * k;
     }
     // the CE target column (one lane of the row)
     if (gce != 0.f && tgt >= col0 && tgt < col0 + 8) {

@@ -93,3 +93,21 @@ def test_nonfinite_tail(gpu, vocab, value):
     x[4, -tail] = value
     t = torch.zeros(6, dtype=torch.long, device=gpu)
     _check_against_torch(x.to(torch.bfloat16), y.to(torch.bfloat16), t)
+
+
+@pytest.mark.parametrize("vocab", [7, 4096, 4103, 16000, 16001, 32000, 40960, 40963, 151936])
+def test_saturated_rows(gpu, vocab):
+    """One token holds all of p and of q to fp32's last digits, so p against q there is rounding: the
+    forward's masses and the backward have to take the same side. p (sign(p - q) - E_p[sign]) is then
+    at most twice the mass outside that token, V e^-30 (the logit's margin: 40 less six sigma of 1.5,
+    rounded up)."""
+    rows = 256
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    x, y = (torch.randn(rows, vocab, device=gpu, generator=g) * 1.5 for _ in range(2))
+    at = torch.randint(0, vocab, (rows, 1), device=gpu, generator=g)
+    for z in (x, y):
+        z.scatter_(1, at, 40 + 30 * torch.rand(rows, 1, device=gpu, generator=g))
+    xin = x.to(torch.bfloat16).requires_grad_()
+    _, l1 = ce_l1_from_logits(xin, at[:, 0], y.to(torch.bfloat16))
+    (grad,) = torch.autograd.grad(l1.sum(), xin)
+    assert grad.abs().max() <= 2 * vocab * np.exp(-30.0)
