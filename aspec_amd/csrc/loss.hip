@@ -103,14 +103,30 @@ __device__ __forceinline__ float scalar_read_bf16(const uint16_t* p) {
 __device__ __forceinline__ float neg_scaled_max(float m) { return -(m * kLog2e); }
 __device__ __forceinline__ float scaled_exp2(float v, float nm) { return fexp2(fmaf(v, kLog2e, nm)); }
 
-// (max, sum) pairs: sum is relative to max. A pair whose max is -inf holds 0 (all masked) or NaN
-// (a NaN logit) and passes through unscaled; +inf maxima give NaN, as softmax does.
+// Sums over part of a row are taken relative to that part's maximum m, with the offset
+// part_offset(m). Its rounding does not cancel at v == m: the exponent there is off by up to half an
+// ulp of m log2e, 64 at m = -2^30. Below that (logits masked with -1e10, -1e30 or the type's lowest
+// value) the sum would overflow, so there the offset is 0 and every exp2 0: the part adds nothing to
+// a row that has anything larger, as in the row's own softmax.
+constexpr float kMaskedBelow = -0x1p30f;
+__device__ __forceinline__ float part_offset(float m) { return m < kMaskedBelow ? 0.f : neg_scaled_max(m); }
+
+// The part's sum relative to a maximum with the offset `to` instead: scaled by the quotient of the
+// two offsets as they were rounded, so a row's sum is that of scaled_exp2 at the row's own offset,
+// whatever maxima its parts met. A masked part holds 0, or NaN of a NaN logit, and is not scaled
+// (the factor may be infinite).
+__device__ __forceinline__ float rebased_sum(float m, float s, float to) {
+  return m < kMaskedBelow ? s : s * fexp2(to - neg_scaled_max(m));
+}
+
+// The exponent that scaled_exp2 has at the maximum itself: the offset's rounding.
+__device__ __forceinline__ float exponent_at_max(float m) { return fmaf(m, kLog2e, neg_scaled_max(m)); }
+
+// Merges two parts' (max, sum) pairs; +inf maxima give NaN, as softmax does.
 __device__ __forceinline__ void merge_max_sum(float& m, float& s, float mo, float so) {
-  const float mn = fmaxf(m, mo);
-  const float a = m == -INFINITY ? s : s * fexp2((m - mn) * kLog2e);
-  const float b = mo == -INFINITY ? so : so * fexp2((mo - mn) * kLog2e);
+  const float mn = fmaxf(m, mo), to = part_offset(mn);
+  s = rebased_sum(m, s, to) + rebased_sum(mo, so, to);
   m = mn;
-  s = a + b;
 }
 
 // Block-wide merge of NP (max, sum) pairs; the result is broadcast to every thread.
@@ -583,9 +599,9 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
     r.max = grow ? cm : r.max;
     if (__any(cm > r.ref + kSlack)) {
       if (cm > r.ref) {
-        r.sum = sum_relative_to(r.ref, r.sum, cm);
+        r.nref = part_offset(cm);
+        r.sum = rebased_sum(r.ref, r.sum, r.nref);
         r.ref = cm;
-        r.nref = neg_scaled_max(cm);
       }
     }
     float e[8];
@@ -627,17 +643,15 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     m[i] = run[i].max;
-    s[i] = sum_relative_to(run[i].ref, run[i].sum, m[i]);
+    s[i] = rebased_sum(run[i].ref, run[i].sum, part_offset(m[i]));
   }
   if (in_tail) {
-    // a lone logit's sum relative to itself: 1, and what merge_max_sum wants of -inf (0) and NaN
-    auto lone = [](float v) { return v == -INFINITY ? 0.f : v == v ? 1.f : v; };
     const float x = bf(xr[tail_at]);
     if (x > m[0]) best = full;
-    merge_max_sum(m[0], s[0], x, lone(x));
+    merge_max_sum(m[0], s[0], x, scaled_exp2(x, part_offset(x)));
     if (has_y) {
       const float y = bf(yr[tail_at]);
-      merge_max_sum(m[1], s[1], y, lone(y));
+      merge_max_sum(m[1], s[1], y, scaled_exp2(y, part_offset(y)));
     }
   }
   const float own_max = m[0];
@@ -724,7 +738,8 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
     block_reduce<4, false>(acc, scratch);
   }
   if (tid == 0) {
-    const float lse = logf(s[0]) + m[0];
+    // less the rounding of the offset, which all of S_x carries
+    const float lse = (logf(s[0]) - kLn2 * exponent_at_max(m[0])) + m[0];
     float* st = a.stats + row * kStats;
     st[0] = m[0]; st[1] = ix; st[2] = m[1]; st[3] = iy;
     st[4] = acc[1]; st[5] = acc[2]; st[6] = acc[3]; st[7] = lse;

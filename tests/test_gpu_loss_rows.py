@@ -111,3 +111,22 @@ def test_saturated_rows(gpu, vocab):
     _, l1 = ce_l1_from_logits(xin, at[:, 0], y.to(torch.bfloat16))
     (grad,) = torch.autograd.grad(l1.sum(), xin)
     assert grad.abs().max() <= 2 * vocab * np.exp(-30.0)
+
+
+@pytest.mark.parametrize("value", [-1e9, -1e10, -1e20, -1e30, torch.finfo(torch.bfloat16).min])
+@pytest.mark.parametrize("vocab", [2055, 8191, 8193, 16383, 40960, 152063])
+def test_large_finite_masks(gpu, vocab, value):
+    """Runs of logits masked with a large finite value at the start, the middle and the end of a row,
+    of a chunk's length and of most of the row, in the draft, the teacher and both."""
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    x, y = (torch.randn(9, vocab, device=gpu, generator=g) * 3 for _ in range(2))
+    mid, most = vocab // 16 * 8, vocab // 64 * 56
+    x[0, :8] = y[1, :8] = value
+    x[2, mid:mid + 64] = y[3, mid:mid + 64] = value
+    x[4, -9:] = y[5, -9:] = value
+    x[6, :most] = y[6, :most] = value
+    x[7, vocab - most:] = value
+    y[8, 8:] = value
+    t = torch.full((9,), vocab // 2, device=gpu)
+    t[2], t[6], t[7], t[4] = 3, vocab - 1, 0, 1
+    _check_against_torch(x.to(torch.bfloat16), y.to(torch.bfloat16), t)
