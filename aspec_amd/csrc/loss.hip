@@ -225,7 +225,7 @@ __device__ __forceinline__ void chunk_exps(const uint4 (&v)[NV], float (&e)[NV *
 #pragma unroll
     for (int k = 0; k < 4; ++k) m = max3_raw(m, lo_bf(w[k]), hi_bf(w[k]));
   }
-  const float nm = m == -INFINITY ? 0.f : neg_scaled_max(m);
+  const float nm = part_offset(m);
   sum = 0.f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -242,8 +242,8 @@ __device__ __forceinline__ void chunk_exps(const uint4 (&v)[NV], float (&e)[NV *
 }
 
 // A (max, sum) pair's sum relative to `to` (>= its max): a pair whose max is -inf passes its sum
-// (0, or NaN from a NaN logit) unscaled; a +inf max against a +inf `to` gives NaN, as softmax
-// does.
+// (0, or NaN from a NaN logit) unscaled, that of a part masked with a large finite value is 0 or
+// NaN too; a +inf max against a +inf `to` gives NaN, as softmax does.
 __device__ __forceinline__ float sum_relative_to(float m, float s, float to) {
   return m == -INFINITY ? s : s * fexp2((m - to) * kLog2e);
 }
@@ -411,7 +411,7 @@ loss_fwd_persistent(LossArgs args) {
     uint32_t key = kNoKey;
     if (ARGMAX) {
       const float M = m[0];
-      if (fabsf(M) >= 0x1p-14f && M < INFINITY && sm[0] == sm[0]) {
+      if (fabsf(M) >= 0x1p-14f && M >= kMaskedBelow && M < INFINITY && sm[0] == sm[0]) {
         // A finite row without NaN whose maximum is not tiny: a thread holding M finds its first
         // maximal element among its exp values, which hold exp2(x log2e - M log2e) (chunk_exps).
         // The maximum gives exactly `emax` (same expression), and any other bf16 logit differs
@@ -424,7 +424,7 @@ loss_fwd_persistent(LossArgs args) {
           key = ((((i0 >> 3) * kWalkThreads + tid) << 3) + (i0 & 7)) | 0x80000000u;
         }
       } else {
-        // a NaN, an infinity, an all -inf row or a tiny maximum: rescan the (cache-resident) row
+        // a NaN, an infinity, an all masked row or a tiny maximum: rescan the (cache-resident) row
         const uint16_t* xr = xbase + row * V;
         for (int64_t i = tid; i < V; i += kWalkThreads)
           key = min(key, argmax_key(bf(xr[i]), M, static_cast<uint32_t>(i)));

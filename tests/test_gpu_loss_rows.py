@@ -114,7 +114,7 @@ def test_saturated_rows(gpu, vocab):
 
 
 @pytest.mark.parametrize("value", [-1e9, -1e10, -1e20, -1e30, torch.finfo(torch.bfloat16).min])
-@pytest.mark.parametrize("vocab", [2055, 8191, 8193, 16383, 40960, 152063])
+@pytest.mark.parametrize("vocab", [2048, 2055, 4096, 8191, 8192, 8193, 16000, 16383, 32000, 40960, 152063])
 def test_large_finite_masks(gpu, vocab, value):
     """Runs of logits masked with a large finite value at the start, the middle and the end of a row,
     of a chunk's length and of most of the row, in the draft, the teacher and both."""
