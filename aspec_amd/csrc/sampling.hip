@@ -20,7 +20,8 @@
 // the boundary's, or equal and its index <= last.
 //
 // The histogram's masses (fp32, any order) only propose a bin: it is taken when the exact mass above
-// it is <= top_p of the total and the mass with it is not, else its neighbour is tried. Masses are
+// it is <= top_p of the total and the mass with it is not, else its neighbour is tried, and no
+// further bin than that: the search over the row follows. Masses are
 // fp32 per token, summed in fp64: over the row in a fixed order, and over a bin's list exactly (its
 // masses lie within e^(1/32) of each other, so at most 2048 of them sum without rounding). So the
 // result does not depend on the order of the atomics. A boundary in the last, open bin or in one of
@@ -38,6 +39,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kBins = 2048;        // bins of 1/32 nat below the maximum: 64 nats, the last one open
 constexpr float kBinsPerNat = 32.f;
 constexpr int kListCap = 2048;     // tokens of the boundary's bin that the list holds
+constexpr int kBinTries = 2;       // bins looked at before the search over the whole row
 constexpr uint32_t kNegInfBits = 0xff80u;  // bf16 -inf: the padding of a row's tail
 
 // per-row, per-side record (8 words); the sampled-L1 row holds draft, teacher, then the masses
@@ -242,8 +244,11 @@ __device__ __forceinline__ uint32_t half_of(const uint32_t (&w)[4], int j) {
 // runs the words through an empty asm in place (no copy, no instruction) and rebuilds the token
 // index from an opaque thread offset, so what a pass derives from them (keys, exp values,
 // indices) is recomputed in that pass instead of being hoisted out of the searches' loops.
+// kWavesPerSimd: the occupancy that the row's own registers allow and the rare searches must not
+// lower (they spill instead): two workgroups of a CU up to 32768 tokens, more for shorter rows.
 template <int NV>
 struct RegRow {
+  static constexpr int kWavesPerSimd = NV == 1 ? 8 : NV == 2 ? 6 : NV <= 8 ? 4 : 2;
   const uint16_t* p;
   uint4 r[NV];
   __device__ __forceinline__ void load(const uint16_t* row, int64_t V) {
@@ -267,6 +272,7 @@ struct RegRow {
 // A row read again from global memory on every pass, for vocabularies beyond the registers' reach
 // (the row stays in the caches between a workgroup's passes).
 struct GlobalRow {
+  static constexpr int kWavesPerSimd = 8;
   const uint16_t* p;
   int64_t V;
   int n;
@@ -655,8 +661,10 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
   __syncthreads();
   const int bin_k = P.use_k ? w.bin_k : kBins;
   int bin = P.use_p ? min(w.bin_p, bin_k) : bin_k;
-  while (true) {
-    if (bin >= kBins - 1) break;
+  // The histogram's bin, then one neighbour, then the search over the row: bounded, because the two
+  // sides of a bin's edge are sums in different orders. In the last digits of top_p they can each
+  // name the other bin, for ever; and there the histogram's fp32 sum can be tens of bins off.
+  for (int tries = 0; tries < kBinTries && bin >= 0 && bin < kBins - 1; ++tries) {
     const float lo = static_cast<float>(bin), hi = static_cast<float>(bin + 1);
     double f = 0.0;
     r.chunks([&](int, int32_t base, const uint32_t (&v)[4]) {
@@ -693,7 +701,6 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
       return st;
     }
     bin += verdict == kHigher ? -1 : 1;
-    if (bin < 0) break;
     __syncthreads();
     if (tid == 0) w.n = 0;
     __syncthreads();
@@ -729,7 +736,8 @@ __device__ __forceinline__ SideStats load_side(const float* src) {
 
 // ---- sampling_logits: the filtered fp32 logits and their gradient ------------------------------
 template <typename Row>
-__global__ void __launch_bounds__(kSampThreads) sampling_fwd_kernel(SampledArgs a) {
+__global__ void __launch_bounds__(kSampThreads) __attribute__((amdgpu_waves_per_eu(Row::kWavesPerSimd)))
+sampling_fwd_kernel(SampledArgs a) {
   __shared__ Work work;
   int ph = 0;
   const int64_t row = blockIdx.x, V = a.V;
@@ -832,7 +840,8 @@ __global__ void __launch_bounds__(kSampThreads) sampling_bwd_kernel(SampledArgs 
 
 // ---- sampled L1 ---------------------------------------------------------------------------------
 template <typename Row>
-__global__ void __launch_bounds__(kSampThreads) sampled_l1_fwd_kernel(SampledArgs a) {
+__global__ void __launch_bounds__(kSampThreads) __attribute__((amdgpu_waves_per_eu(Row::kWavesPerSimd)))
+sampled_l1_fwd_kernel(SampledArgs a) {
   __shared__ Work work;
   int ph = 0;
   const int64_t row = blockIdx.x;

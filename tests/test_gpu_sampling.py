@@ -110,6 +110,30 @@ def test_boundary_bin_edges(gpu, vocab, ties):
     assert int(torch.isfinite(sampling_logits(x[:1], (1.0, 0.5, -1))).sum()) == keep
 
 
+@pytest.mark.parametrize("vocab", [17, 8192, 32000, 98304, 151936])
+@pytest.mark.parametrize("top_p", [1 - 2**-24, 1 - 7 * 2**-24, 1 - 2**-17, 0.99999])
+def test_top_p_in_the_last_digits(gpu, vocab, top_p):
+    """top_p within rounding of 1, where the histogram's sums and the exact ones part: the search ends,
+    keeps a prefix of the order, and its length is that of a top_p within 1e-6 (fp32 exp values,
+    each within 5e-7) of the given one; twice the same bits."""
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    x = torch.cat((_rows(gpu, 6, vocab, vocab), (torch.randn(6, vocab, device=gpu, generator=g) * 6).to(torch.bfloat16)))
+    xn = _np(x)
+    for temperature in (1.0, 0.7):
+        out = sampling_logits(x, (temperature, top_p, -1))
+        assert torch.equal(out, sampling_logits(x, (temperature, top_p, -1)))
+        s = S.scaled_values(xn, (temperature, 1.0, -1)).astype(np.float64)
+        kept = torch.isfinite(out).cpu().numpy()
+        for r in range(x.shape[0]):
+            order = np.argsort(-s[r], kind="stable")
+            order = order[np.isfinite(s[r][order])]
+            n = int(kept[r].sum())
+            assert kept[r][order[:n]].all(), (temperature, r)
+            e = np.exp(s[r][order] - s[r].max())
+            before = (np.cumsum(e) - e) / e.sum()
+            assert (before <= top_p - 1e-6).sum() <= n <= (before <= top_p + 1e-6).sum(), (temperature, r)
+
+
 @pytest.mark.parametrize("vocab", [4097, 32000, 151936])
 def test_sampling_logits_gradient(gpu, vocab):
     x = _rows(gpu, 5, vocab, 3).requires_grad_()
