@@ -21,11 +21,11 @@
 //
 // The histogram's masses (fp32, any order) only propose a bin: it is taken when the exact mass above
 // it is <= top_p of the total and the mass with it is not, else its neighbour is tried, and no
-// further bin than that: the search over the row follows. Masses are
-// fp32 per token, summed in fp64: over the row in a fixed order, and over a bin's list exactly (its
-// masses lie within e^(1/32) of each other, so at most 2048 of them sum without rounding). So the
-// result does not depend on the order of the atomics. A boundary in the last, open bin or in one of
-// more than 2048 tokens (all-equal rows) is found by binary searches over the whole row instead.
+// further bin than that. Masses are fp32 per token, summed in fp64: over the row in a fixed order, and
+// over a bin's list exactly (its masses lie within e^(1/32) of each other, so at most 2048 of them sum
+// without rounding). A boundary in the last, open bin or in one of more than 2048 tokens (flat rows,
+// few distinct values) is found in passes over the row's 16-bit keys instead (search_row), where sums
+// in a fixed order decide as well. So the result does not depend on the order of the atomics.
 #include <cmath>
 
 #include "common.h"
@@ -181,6 +181,10 @@ __device__ __forceinline__ double uniform(double v) {
   return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float uniform(float v) { return __uint_as_float(uniform(__float_as_uint(v))); }
+
 // Two slot sets used alternately: the barrier of the call in between separates the reads of one
 // call from the writes of the call after next. Every thread adds the eight waves' slots in one
 // fixed pairing.
@@ -214,7 +218,7 @@ __device__ __forceinline__ float block_max(float v, bool bad, bool& any_bad, Red
     any_bad |= o != o;
     m = fmax(m, o);
   }
-  return static_cast<float>(uniform(m));
+  return uniform(static_cast<float>(m));
 }
 
 // ---- rows -------------------------------------------------------------------------------------
@@ -242,8 +246,8 @@ __device__ __forceinline__ uint32_t half_of(const uint32_t (&w)[4], int j) {
 
 // A row held in registers (NV chunks of packed bf16 per thread: up to 98304 tokens). Each pass
 // runs the words through an empty asm in place (no copy, no instruction) and rebuilds the token
-// index from an opaque thread offset, so what a pass derives from them (keys, exp values,
-// indices) is recomputed in that pass instead of being hoisted out of the searches' loops.
+// index from an opaque thread offset, so what a pass derives from them (exp values, bins, indices)
+// is recomputed in that pass instead of being kept in registers from the one before.
 // kWavesPerSimd: the occupancy that the row's own registers allow and the rare searches must not
 // lower (they spill instead): two workgroups of a CU up to 32768 tokens, more for shorter rows.
 template <int NV>
@@ -257,6 +261,7 @@ struct RegRow {
     for (int c = 0; c < NV; ++c)
       r[c] = row_chunk(row, V, (static_cast<int64_t>(c) * kSampThreads + threadIdx.x) * 8);
   }
+  __device__ __forceinline__ uint4 first() const { return r[0]; }
   template <typename G>
   __device__ __forceinline__ void chunks(G&& g) {
     const int32_t t8 = opaque_t8();
@@ -280,6 +285,7 @@ struct GlobalRow {
     p = row, V = V_;
     n = static_cast<int>((V + 8LL * kSampThreads - 1) / (8LL * kSampThreads));
   }
+  __device__ __forceinline__ uint4 first() const { return row_chunk(p, V, static_cast<int64_t>(threadIdx.x) * 8); }
   template <typename G>
   __device__ __forceinline__ void chunks(G&& g) {
     const int32_t t8 = static_cast<int32_t>(threadIdx.x) * 8;
@@ -323,27 +329,34 @@ struct Work {
   Red red;
   float mass[kBins + kWave];  // past kBins: where the last bin's adds go, a word per lane, never read
   uint32_t count[kBins + kWave];
-  uint32_t key[kListCap];  // the list: x_key and index of the tokens of the bin looked at
-  int32_t idx[kListCap];
+  union {
+    struct {
+      uint32_t key[kListCap];  // the list: x_key and index of the tokens of the bin looked at
+      int32_t idx[kListCap];
+    };
+    double hist[kBins];  // the row's search: mass or count per group of keys
+  };
+  double part[kWave];
   float wave_mass[kSampWaves];
   uint32_t wave_count[kSampWaves];
   uint32_t n;        // tokens appended to the list
+  uint32_t level;    // waves whose first tokens lie within three bins
   int32_t bin_p, bin_k;
   int32_t verdict;   // what the list's wave found: see Verdict
   uint32_t okey;
   int32_t last;
   double z;
 };
-enum Verdict { kFound, kHigher, kLower };
+enum Verdict { kFound, kLower };
 
 // The distance of a sort value below the maximum in bins, as a float: its integer part is the bin
 // (the last bin takes everything beyond). A function of the scaled value, so tokens that tie share
 // a bin.
 __device__ __forceinline__ float bin_of(float u) { return fminf(-u * kBinsPerNat, static_cast<float>(kBins - 1)); }
 
-// The end of the search on one bin's list, by one wave: `above` is the exact mass and `before` the
-// count of the tokens in higher bins, lim = top_p times the row's mass; use_k says whether top_k's
-// boundary lies in this bin.
+// The end of the search on one bin's list, by one wave: `above` (<= lim with top-p) is the exact mass
+// and `before` the count of the tokens in higher bins, lim = top_p times the row's mass; use_k says
+// whether top_k's boundary lies in this bin.
 __device__ __forceinline__ void search_list(Work& w, int n, const RowCtx& cx, bool use_p, double lim, double above,
                                             bool use_k, int64_t top_k, int64_t before) {
   const int lane = threadIdx.x & 63;
@@ -361,10 +374,6 @@ __device__ __forceinline__ void search_list(Work& w, int n, const RowCtx& cx, bo
   mass = wave_sum_d(mass);
   bool have_p = false;
   if (use_p) {
-    if (above > lim) {  // the top-p boundary lies in a higher bin
-      if (lane == 0) w.verdict = kHigher;
-      return;
-    }
     have_p = above + mass > lim;
     if (!have_p && !use_k) {
       if (lane == 0) w.verdict = kLower;
@@ -456,111 +465,272 @@ __device__ __forceinline__ void search_list(Work& w, int n, const RowCtx& cx, bo
   }
 }
 
-// The support by binary searches over the whole row (16-bit keys, then token indices): for a
-// boundary that the list cannot hold, read from the caches in rolled loops (unrolled over a row's
-// registers, this rare path was most of the file's code). `total` is the row's mass.
-__device__ __forceinline__ void search_row(GlobalRow& r, int64_t V, const SideParams& P, const RowCtx& cx, double total,
-                                        SideStats& st, Red& red, int& ph) {
-  bool have_p = false, have_k = false;
-  uint32_t okey_p = 0, okey_k = 0;
-  int64_t n_p = 0, c_p = 0, n_k = 0, c_k = 0;
-  if (P.use_p) {
-    const double lim = static_cast<double>(P.top_p) * total;
-    uint32_t lo = 0, hi = 0xffffu;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi) >> 1;
-      double f = 0.0;
-      for_each(r, [&](uint32_t h, int32_t) { f += x_key(h) > mid ? e_of(bf16f(h), cx) : 0.0f; }, [&] { fence(f); });
-      if (block_sum(f, red, ph) <= lim) hi = mid;
-      else lo = mid + 1;
-    }
-    if (lo != 0) {  // key 0 (a negative NaN) is never present: lo == 0 keeps every token
-      have_p = true;
-      const float xb = bf16f(x_bits_of_key(lo));
-      okey_p = ord_key(ord_of(xb, cx));
-      const float eb = e_of(xb, cx);
-      double f = 0.0;
-      uint32_t c = 0;
-      for_each(r, [&](uint32_t h, int32_t) {
-        const uint32_t k = ord_key(ord_of(bf16f(h), cx));
-        f += k > okey_p ? e_of(bf16f(h), cx) : 0.0f;
-        c += k == okey_p ? 1u : 0u;
-      }, [&] { fence(f, c); });
-      const double above = block_sum(f, red, ph);
-      c_p = block_count(c, red, ph);
-      // the j-th tie (0-based, index order) has mass above + j * eb before it
-      if (eb > 0.0f) {
-        const double q = floor((lim - above) / static_cast<double>(eb));
-        n_p = q + 1.0 >= static_cast<double>(c_p) ? c_p : static_cast<int64_t>(q) + 1;
-      } else {
-        n_p = c_p;
-      }
-    }
+// The first lane at which base + the sum of the lanes' values up to it exceeds target, and that sum
+// without the lane; -1 and the whole sum if there is none.
+struct First {
+  int at;
+  double before;
+};
+__device__ __forceinline__ First first_lane_over(double own, double base, double target) {
+  double inc = own;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const double from = __shfl_up(inc, o);
+    if ((threadIdx.x & 63) >= o) inc += from;
   }
-  if (P.use_k) {  // 0 < top_k < V: the boundary is a present key
-    have_k = true;
-    uint32_t lo = 0, hi = 0xffffu;
+  const uint64_t over = __ballot(base + inc > target);
+  if (!over) return First{-1, base + uniform(__shfl(inc, kWave - 1))};
+  const int at = __ffsll(static_cast<unsigned long long>(over)) - 1;
+  return First{at, base + uniform(__shfl(inc - own, at))};
+}
+
+// The same over n entries of w.hist, every wave by itself: up to a lane each; or kBins of them, first
+// over the sums of 32.
+__device__ __forceinline__ First first_entry_over(int n, double base, double target, Work& w) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (n <= kWave) return first_lane_over(lane < n ? w.hist[lane] : 0.0, base, target);
+  constexpr int kPer = kBins / kWave;
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < kBins / kSampThreads; ++i) s += w.hist[tid * (kBins / kSampThreads) + i];
+#pragma unroll
+  for (int o = 1; o < kSampThreads / kWave; o <<= 1) s += __shfl_xor(s, o);
+  if (tid % (kSampThreads / kWave) == 0) w.part[tid / (kSampThreads / kWave)] = s;
+  __syncthreads();
+  const First part = first_lane_over(w.part[lane], base, target);
+  if (part.at < 0) return part;
+  const First f = first_lane_over(lane < kPer ? w.hist[part.at * kPer + lane] : 0.0, part.before, target);
+  // (-1: the sums' rounding differs; any entry of the part is as good a proposal)
+  return First{part.at * kPer + max(f.at, 0), f.at < 0 ? part.before : f.before};
+}
+
+// Keys of a row to look for a boundary in, and the mass (top-p) or count (top-k) of the tokens above.
+struct KeyRange {
+  uint32_t lo, hi;
+  double above;
+};
+constexpr KeyRange kAllKeys = {0u, 0xffffu, 0.0};
+
+// The keys of the tokens in a bin: bin_of falls as the key rises.
+__device__ __forceinline__ KeyRange keys_of_bin(int bin, const RowCtx& cx, double above) {
+  uint32_t edge[2];  // the lowest keys in bins <= bin and <= bin - 1
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    uint32_t lo = x_key(kNegInfBits), hi = x_key(kNegInfBits ^ 0x8000u);
     while (lo < hi) {
       const uint32_t mid = (lo + hi) >> 1;
-      uint32_t cnt = 0;
-      for_each(r, [&](uint32_t h, int32_t) { cnt += x_key(h) > mid ? 1u : 0u; }, [&] { fence(cnt); });
-      if (block_count(cnt, red, ph) <= P.top_k - 1) hi = mid;
+      if (static_cast<int>(bin_of(u_of(bf16f(x_bits_of_key(mid)), cx))) <= bin - i) hi = mid;
       else lo = mid + 1;
     }
-    okey_k = ord_key(ord_of(bf16f(x_bits_of_key(lo)), cx));
-    uint32_t a = 0, c = 0;
+    edge[i] = lo;
+  }
+  return KeyRange{uniform(edge[0]), uniform(bin == 0 ? 0xffffu : max(edge[0], edge[1] - 1)), above};
+}
+
+// The key in a range, or below it, at which mass or count pass `target`, from fp64 sums over groups of
+// keys (added in any order: a proposal in the last digits): a pass for up to 2048 keys, or two. A thread
+// adds up tokens of one group before it goes to LDS, so rows of few distinct values (masked, all
+// equal) do not queue up on one address.
+__device__ __forceinline__ uint32_t likely_key(GlobalRow& r, const RowCtx& cx, KeyRange range, bool by_mass,
+                                               double target, Work& w) {
+  while (true) {
+    int shift = 0;
+    while (((range.hi - range.lo) >> shift) >= static_cast<uint32_t>(kBins)) ++shift;
+    const int groups = static_cast<int>((range.hi - range.lo) >> shift) + 1;
+    __syncthreads();
+    for (int i = threadIdx.x; i < (groups <= kWave ? kWave : kBins); i += kSampThreads) w.hist[i] = 0.0;
+    __syncthreads();
+    uint32_t group = 0;
+    double sum = 0.0;
+    auto flush = [&] {
+      if (sum > 0.0) __hip_atomic_fetch_add(&w.hist[group], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      sum = 0.0;
+    };
     for_each(r, [&](uint32_t h, int32_t) {
-      const uint32_t k = ord_key(ord_of(bf16f(h), cx));
-      a += k > okey_k ? 1u : 0u;
-      c += k == okey_k ? 1u : 0u;
-    }, [&] { fence(a, c); });
-    const int64_t above = block_count(a, red, ph);
-    c_k = block_count(c, red, ph);
-    n_k = P.top_k - above;
-  }
-  // both filters keep a prefix of the order: the shorter one wins
-  uint32_t okey = 0;
-  int64_t n = 0, cnt = 0;
-  if (have_p && (!have_k || okey_p > okey_k)) {
-    okey = okey_p, n = n_p, cnt = c_p;
-  } else if (have_k && (!have_p || okey_k > okey_p)) {
-    okey = okey_k, n = n_k, cnt = c_k;
-  } else if (have_p && have_k) {
-    okey = okey_p, n = n_p < n_k ? n_p : n_k, cnt = c_p;
-  }
-  st.okey = okey;
-  st.last = 0x7fffffff;
-  if (!have_p && !have_k) {
-    st.flags |= kFlagAll;
-  } else if (n < cnt) {
-    // index of the n-th tie: the smallest j with n ties at indices <= j
-    int64_t lo = 0, hi = V - 1;
-    while (lo < hi) {
-      const int64_t mid = (lo + hi) >> 1;
-      uint32_t c = 0;
-      for_each(r, [&](uint32_t h, int32_t idx) {
-        c += ((idx <= mid) & (ord_key(ord_of(bf16f(h), cx)) == okey)) ? 1u : 0u;
-      }, [&] { fence(c); });
-      if (block_count(c, red, ph) >= n) hi = mid;
-      else lo = mid + 1;
+      const uint32_t k = x_key(h);
+      if (k >= range.lo && k <= range.hi) {
+        const uint32_t g = (range.hi - k) >> shift;
+        if (g != group) flush();
+        group = g;
+        sum += by_mass ? e_of(bf16f(h), cx) : 1.0f;
+      }
+      fence(group, sum);  // token by token: this path is rare, its registers are every row's
+    }, [] {});
+    flush();
+    __syncthreads();
+    const First f = first_entry_over(groups, range.above, target, w);
+    if (f.at < 0) {
+      if (range.lo == 0) return 0;
+      range = KeyRange{0u, range.lo - 1, f.before};
+      continue;
     }
-    st.last = static_cast<int32_t>(lo);
+    const uint32_t top = range.hi - (static_cast<uint32_t>(f.at) << shift);
+    if (shift == 0) return top;
+    range = KeyRange{max(range.lo, top - ((1u << shift) - 1)), top, f.before};
   }
-  double z = 0.0;
-  const Support sup = support_of(st);
-  for_each(r, [&](uint32_t h, int32_t idx) {
-    const float x = bf16f(h);
-    z += kept(sup, ord_of(x, cx), idx) ? e_of(x, cx) : 0.0f;
-  }, [&] { fence(z); });
-  st.zinv = static_cast<float>(1.0 / block_sum(z, red, ph));
+}
+
+// One pass around a boundary at x_key k: the mass or count of the keys above k and from k on, and
+// of the boundary's ties in scaled values the mass and count above them and their number, this also
+// per step of 4096 tokens (V > 2^18: several steps) in w.count. Sums in a fixed order.
+struct Around {
+  double gt, ge, mass;
+  int64_t over, same;
+};
+constexpr int kStepShift = 12;  // log2 of the tokens a workgroup's chunks cover
+static_assert(kSampThreads * 8 == 1 << kStepShift, "one chunk per thread");
+// (log2 of the tokens that an entry of w.count covers: at most a lane's worth of entries)
+__device__ __forceinline__ int tie_shift(int64_t V) {
+  int shift = kStepShift;
+  while (((V - 1) >> shift) >= kWave) ++shift;
+  return shift;
+}
+
+__device__ __forceinline__ Around around(GlobalRow& r, uint32_t k, const RowCtx& cx, bool by_mass, Work& w, int& ph) {
+  const uint32_t o = ord_key(ord_of(bf16f(x_bits_of_key(k)), cx));
+  const int shift = tie_shift(r.V);
+  __syncthreads();
+  if (threadIdx.x < kWave) w.count[threadIdx.x] = 0u;
+  __syncthreads();
+  double gt = 0.0, ge = 0.0, mass = 0.0;
+  uint32_t over = 0, same = 0;
+  r.chunks([&](int, int32_t base, const uint32_t (&v)[4]) {
+    uint32_t ties = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t h = half_of(v, j), key = x_key(h);
+      const uint32_t oi = ord_key(ord_of(bf16f(h), cx));
+      const float e = e_of(bf16f(h), cx), by = by_mass ? e : 1.0f;
+      gt += key > k ? by : 0.0f;
+      ge += key >= k ? by : 0.0f;
+      mass += oi > o ? e : 0.0f;
+      over += oi > o ? 1u : 0u;
+      ties += oi == o ? 1u : 0u;
+      fence(gt, ge, mass, over, ties);
+    }
+    same += ties;
+    const uint32_t all = wave_sum_u(ties);
+    if ((threadIdx.x & 63) == 0 && all) atomicAdd(&w.count[base >> shift], all);
+  });
+  Around a;
+  a.gt = block_sum(gt, w.red, ph);
+  a.ge = block_sum(ge, w.red, ph);
+  a.mass = block_sum(mass, w.red, ph);
+  a.over = block_count(over, w.red, ph);
+  a.same = block_count(same, w.red, ph);
+  return a;
+}
+
+// The index of the keep-th tie of the boundary that around() last saw: its step from w.count, then
+// a scan of that step's tokens.
+__device__ __forceinline__ int32_t tie_index(const GlobalRow& r, uint32_t o, int64_t keep, const RowCtx& cx, Work& w) {
+  const int tid = threadIdx.x, shift = tie_shift(r.V);
+  const First f = first_lane_over(static_cast<double>(w.count[tid & 63]), 0.0, static_cast<double>(keep - 1));
+  int64_t left = keep - static_cast<int64_t>(f.before);  // 1-based in the group
+  const int64_t begin = static_cast<int64_t>(f.at) << shift, end = begin + (int64_t{1} << shift);
+  for (int64_t start = begin; start < end; start += 1 << kStepShift) {
+    const int32_t base = static_cast<int32_t>(start) + tid * 8;
+    const uint4 c = row_chunk(r.p, r.V, base);
+    const uint32_t v[4] = {c.x, c.y, c.z, c.w};
+    uint32_t own = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) own += ord_key(ord_of(bf16f(half_of(v, j)), cx)) == o ? 1u : 0u;
+    uint32_t upto = own;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const uint32_t from = __shfl_up(upto, d);
+      if ((tid & 63) >= d) upto += from;
+    }
+    if ((tid & 63) == 63) w.wave_count[tid >> 6] = upto;
+    __syncthreads();
+    uint32_t total = 0;
+#pragma unroll
+    for (int i = 0; i < kSampWaves; ++i) {
+      if (i < (tid >> 6)) upto += w.wave_count[i];
+      total += w.wave_count[i];
+    }
+    if (left > upto - own && left <= upto) {
+      int64_t n = left - (upto - own);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (ord_key(ord_of(bf16f(half_of(v, j)), cx)) == o && --n == 0) w.last = base + j;
+    }
+    __syncthreads();
+    left -= total;
+    if (left <= 0) break;
+  }
+  return w.last;
+}
+
+// The support from passes over the row in global memory (rolled loops: unrolled over a row's
+// registers this rare path was most of the file's code), for a boundary that the list cannot hold.
+// A key per filter is proposed from a histogram, and one exact pass around it shows that the mass (or
+// count) above is <= the limit and with it is not; else a binary search over the 16-bit keys goes on
+// from what that pass showed. in_p and in_k: where to look first. Two or three passes, against the
+// some thirty of binary searches over keys and indices, in registers up to 98304 tokens:
+// sampling_logits of 512 x 98304, sigma 0.3, top-p 877 -> 509 us; 400 x 151936 all equal 1458 -> 311;
+// 1024 x 32000 with 41 tokens not masked, top-k 50, 472 -> 154; 2048 x 2560 all equal 139 -> 76.
+__device__ __forceinline__ void search_row(GlobalRow& r, const SideParams& P, const RowCtx& cx, double total,
+                                           KeyRange in_p, KeyRange in_k, SideStats& st, Work& w, int& ph) {
+  const double lim = uniform(static_cast<double>(P.top_p) * total);
+  uint32_t key = 0, okey = 0, seen = 0;  // the shorter prefix's boundary, and the key last looked at
+  int64_t keep = 0, ties = 0;
+  double mass = 0.0;
+#pragma unroll 1
+  for (int filter = 0; filter < 2; ++filter) {  // top-k, then top-p
+    const bool by_mass = filter == 1;
+    if (!(by_mass ? P.use_p : P.use_k)) continue;
+    uint32_t lo = 0, hi = 0xffffu;  // the smallest key with at most `target` above it lies here
+    KeyRange in = {by_mass ? in_p.lo : in_k.lo, by_mass ? in_p.hi : in_k.hi, by_mass ? in_p.above : in_k.above};
+    if (by_mass && P.use_k) {
+      // top-p matters where it ends before top-k's last token
+      if (mass + static_cast<double>(e_of(bf16f(x_bits_of_key(key)), cx)) * static_cast<double>(keep - 1) <= lim) break;
+      lo = key;
+    }
+    const double target = by_mass ? lim : uniform(static_cast<double>(P.top_k - 1));
+    uint32_t mid = max(likely_key(r, cx, in, by_mass, target, w), lo);
+    Around a;
+    while (true) {
+      a = around(r, mid, cx, by_mass, w, ph);
+      if (a.gt > target && mid < hi) lo = mid + 1;
+      else if (a.ge <= target && mid > lo) hi = mid - 1;
+      else break;
+      mid = (lo + hi) >> 1;
+    }
+    seen = mid;
+    const float xb = bf16f(x_bits_of_key(mid));
+    const uint32_t o = uniform(ord_key(ord_of(xb, cx)));
+    int64_t n = a.same;
+    if (by_mass) {
+      const float eb = e_of(xb, cx);
+      if (eb > 0.0f) {
+        // the j-th tie (0-based, index order) has mass a.mass + j * eb before it
+        const double q = floor((lim - a.mass) / static_cast<double>(eb));
+        if (q + 1.0 < static_cast<double>(a.same)) n = static_cast<int64_t>(uniform(q)) + 1;
+      }
+    } else {
+      n = P.top_k - a.over;
+    }
+    // both filters keep a prefix of the order: the shorter one wins
+    if (ties == 0 || o > okey || (o == okey && n < keep)) key = mid, okey = o, keep = n, ties = a.same, mass = a.mass;
+  }
+  st.okey = uniform(okey);
+  st.last = 0x7fffffff;
+  if (keep < ties) {
+    if (seen != key) around(r, key, cx, false, w, ph);
+    st.last = uniform(tie_index(r, okey, keep, cx, w));
+  }
+  const float eb = e_of(bf16f(x_bits_of_key(key)), cx);
+  st.zinv = uniform(static_cast<float>(1.0 / (mass + static_cast<double>(eb) * static_cast<double>(keep))));
 }
 
 // One side's support and normaliser. Rows with a NaN or no finite maximum get kFlagNaN (the
 // reference's softmax gives NaN there).
-template <typename Row>
+template <bool FILTER, typename Row>
 __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const SideParams P, Work& w, int& ph) {
   const int tid = threadIdx.x;
   SideStats st = {};
+  if (tid == 0) w.level = 0;
   float mx = -INFINITY;
   uint32_t mag = 0;  // the largest magnitude bits: above 0x7f80 is a NaN
   for_each(r, [&](uint32_t h, int32_t) {
@@ -577,12 +747,23 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     return st;
   }
   const RowCtx cx{m, st.rcp_t, P.temp != 0};
-  const bool filter = P.use_p || P.use_k;
+  const bool filter = FILTER && (P.use_p || P.use_k);
   if (filter) {
     for (int i = tid; i < kBins; i += kSampThreads) w.mass[i] = 0.0f, w.count[i] = 0u;
     if (tid == 0) w.n = 0, w.bin_p = kBins - 1, w.bin_k = kBins - 1;
+    // A level row, most of whose first tokens lie within three bins: its adds would queue up on these,
+    // and the list could not hold their bin. The histogram stays empty and the row's search decides.
+    const uint4 c = r.first();
+    const uint32_t v[4] = {c.x, c.y, c.z, c.w};
+    const float b0 = uniform(bin_of(u_of(bf16f(half_of(v, 0)), cx)));
+    bool near = b0 < kBins - 1;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) near &= fabsf(bin_of(u_of(bf16f(half_of(v, j)), cx)) - b0) < 3.0f;
+    if (__popcll(__ballot(near)) >= 48 && (tid & 63) == 0) atomicAdd(&w.level, 1u);
     __syncthreads();
   }
+  const bool level = filter && V > kListCap && uniform(w.level) > kSampWaves / 2;
+  const bool hist_p = P.use_p && !level, hist_k = P.use_k && !level;
   // the total mass, the tokens equal to the maximum and the histogram
   double se = 0.0;
   uint32_t nm = 0;
@@ -600,12 +781,12 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
       const int b = static_cast<int>(bin_of(u_of(x, cx)));
       at[j] = b < kBins - 1 ? b : sink;
     }
-    if (P.use_p && base < V) {
+    if (hist_p && base < V) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         __hip_atomic_fetch_add(&w.mass[at[j]], e[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    if (P.use_k && base < V) {
+    if (hist_k && base < V) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         __hip_atomic_fetch_add(&w.count[at[j]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -613,15 +794,15 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     fence(se, nm);
   });
   const double total = block_sum(se, w.red, ph);  // its barrier also completes the histogram
-  st.nmax = static_cast<int32_t>(block_count(nm, w.red, ph));
-  if (!filter) {
+  st.nmax = uniform(static_cast<int32_t>(block_count(nm, w.red, ph)));
+  if (!FILTER || !filter) {
     st.flags |= kFlagAll;
     st.last = 0x7fffffff;
-    st.zinv = static_cast<float>(1.0 / total);
+    st.zinv = uniform(static_cast<float>(1.0 / total));
     return st;
   }
   // The bins that hold the top-p and top-k boundaries: thread t scans bins 4t .. 4t+3.
-  const double lim = static_cast<double>(P.top_p) * total;
+  const double lim = uniform(static_cast<double>(P.top_p) * total);
   constexpr int kPer = kBins / kSampThreads;
   float own_m[kPer];
   uint32_t own_c[kPer];
@@ -646,7 +827,11 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
   __syncthreads();
   float run_m = inc_m - sum_m;
   uint32_t run_c = inc_c - sum_c;
-  for (int i = 0; i < (tid >> 6); ++i) run_m += w.wave_mass[i], run_c += w.wave_count[i];
+#pragma unroll
+  for (int i = 0; i < kSampWaves - 1; ++i) {
+    run_m += i < (tid >> 6) ? w.wave_mass[i] : 0.0f;
+    run_c += i < (tid >> 6) ? w.wave_count[i] : 0u;
+  }
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     run_m += own_m[i];
@@ -659,13 +844,20 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
     }
   }
   __syncthreads();
-  const int bin_k = P.use_k ? w.bin_k : kBins;
-  int bin = P.use_p ? min(w.bin_p, bin_k) : bin_k;
+  const int bin_k = uniform(P.use_k ? w.bin_k : kBins);
+  int bin = uniform(P.use_p ? min(w.bin_p, bin_k) : bin_k);
+  const int64_t before_k = P.use_k ? static_cast<int64_t>(uniform(w.count[min(bin_k, kBins - 1)])) : 0;
+  KeyRange in_p = kAllKeys;
   // The histogram's bin, then one neighbour, then the search over the row: bounded, because the two
   // sides of a bin's edge are sums in different orders. In the last digits of top_p they can each
   // name the other bin, for ever; and there the histogram's fp32 sum can be tens of bins off.
   for (int tries = 0; tries < kBinTries && bin >= 0 && bin < kBins - 1; ++tries) {
     const float lo = static_cast<float>(bin), hi = static_cast<float>(bin + 1);
+    // A bin that the histogram shows to hold more tokens than the list is only summed up: its tokens'
+    // appends, one counter for all, would take longer than the search they cannot help.
+    const float crowd = P.use_p ? w.mass[bin] * __builtin_amdgcn_exp2f(lo * (kLog2e / kBinsPerNat))
+                                : static_cast<float>(w.count[bin + 1] - w.count[bin]);
+    const bool crowded = uniform(crowd) > 1.01f * kListCap;
     double f = 0.0;
     r.chunks([&](int, int32_t base, const uint32_t (&v)[4]) {
       uint32_t in_bin = 0;
@@ -676,6 +868,7 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
         f += b < lo ? e_of(x, cx) : 0.0f;
         in_bin |= ((b >= lo) & (b < hi)) ? 1u << j : 0u;
       }
+      if (crowded) in_bin = 0;
       for (; in_bin; in_bin &= in_bin - 1) {  // few tokens of a row
         const int j = __ffs(in_bin) - 1;
         const uint32_t word = (j & 4) ? ((j & 2) ? v[3] : v[2]) : ((j & 2) ? v[1] : v[0]);
@@ -686,28 +879,34 @@ __device__ __forceinline__ SideStats compute_support(Row& r, int64_t V, const Si
       fence(f);
     });
     const double above = block_sum(f, w.red, ph);  // its barrier also completes the list
-    const uint32_t n = w.n;
-    if (n > kListCap) break;
-    if (tid < kWave)
-      search_list(w, static_cast<int>(n), cx, P.use_p, lim, above, bin == bin_k, P.top_k,
-                  P.use_k ? static_cast<int64_t>(w.count[bin]) : 0);
-    __syncthreads();
-    const int verdict = w.verdict;
-    if (verdict == kFound) {
-      st.okey = w.okey;
-      st.last = w.last;
-      st.zinv = static_cast<float>(1.0 / w.z);
-      __syncthreads();  // w is reused by the row's other side
-      return st;
+    const uint32_t n = uniform(w.n);
+    const bool higher = P.use_p && above > lim;
+    if (!higher) {
+      if (crowded || n > kListCap) {
+        in_p = keys_of_bin(bin, cx, above);
+        break;
+      }
+      if (tid < kWave)
+        search_list(w, static_cast<int>(n), cx, P.use_p, lim, above, bin == bin_k, P.top_k, before_k);
+      __syncthreads();
+      if (uniform(w.verdict) == kFound) {
+        st.okey = uniform(w.okey);
+        st.last = uniform(w.last);
+        st.zinv = uniform(static_cast<float>(1.0 / w.z));
+        __syncthreads();  // w is reused by the row's other side
+        return st;
+      }
     }
-    bin += verdict == kHigher ? -1 : 1;
+    bin += higher ? -1 : 1;
     __syncthreads();
     if (tid == 0) w.n = 0;
     __syncthreads();
   }
+  const KeyRange in_k = P.use_k && bin_k < kBins - 1 ? keys_of_bin(bin_k, cx, static_cast<double>(before_k)) : kAllKeys;
   GlobalRow again;
   again.load(r.p, V);
-  search_row(again, V, P, cx, total, st, w.red, ph);
+  search_row(again, P, cx, total, in_p, in_k, st, w, ph);
+  __syncthreads();  // w is reused by the row's other side
   return st;
 }
 
@@ -735,7 +934,7 @@ __device__ __forceinline__ SideStats load_side(const float* src) {
 }
 
 // ---- sampling_logits: the filtered fp32 logits and their gradient ------------------------------
-template <typename Row>
+template <typename Row, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) __attribute__((amdgpu_waves_per_eu(Row::kWavesPerSimd)))
 sampling_fwd_kernel(SampledArgs a) {
   __shared__ Work work;
@@ -744,7 +943,7 @@ sampling_fwd_kernel(SampledArgs a) {
   const SideParams px = a.px;
   Row r;
   r.load(a.x + row * V, V);
-  const SideStats s = compute_support(r, V, px, work, ph);
+  const SideStats s = compute_support<FILTER>(r, V, px, work, ph);
   const RowCtx cx = ctx_of(s);
   const Support sup = support_of(s);
   float* out = a.out + row * V;
@@ -839,7 +1038,7 @@ __global__ void __launch_bounds__(kSampThreads) sampling_bwd_kernel(SampledArgs 
 }
 
 // ---- sampled L1 ---------------------------------------------------------------------------------
-template <typename Row>
+template <typename Row, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) __attribute__((amdgpu_waves_per_eu(Row::kWavesPerSimd)))
 sampled_l1_fwd_kernel(SampledArgs a) {
   __shared__ Work work;
@@ -865,9 +1064,9 @@ sampled_l1_fwd_kernel(SampledArgs a) {
   const uint16_t* yr = a.y + yrow * V;
   Row r;
   r.load(yr, V);
-  const SideStats sy = compute_support(r, V, py, work, ph);
+  const SideStats sy = compute_support<FILTER>(r, V, py, work, ph);
   r.load(xr, V);
-  const SideStats sx = compute_support(r, V, px, work, ph);
+  const SideStats sx = compute_support<FILTER>(r, V, px, work, ph);
   const bool nan_row = ((sx.flags | sy.flags) & kFlagNaN) != 0;
   double l1 = 0.0, pos = 0.0, neg = 0.0, zero = 0.0;
   if (!nan_row) {
@@ -977,16 +1176,24 @@ int chunks_for(int64_t V) {
   return 0;
 }
 
-#define ASPEC_SAMPLING_DISPATCH(KERNEL, NV, ...)                                                    \
-  switch (NV) {                                                                                     \
-    case 1: hipLaunchKernelGGL(KERNEL<RegRow<1>>, __VA_ARGS__); break;                               \
-    case 2: hipLaunchKernelGGL(KERNEL<RegRow<2>>, __VA_ARGS__); break;                               \
-    case 4: hipLaunchKernelGGL(KERNEL<RegRow<4>>, __VA_ARGS__); break;                               \
-    case 8: hipLaunchKernelGGL(KERNEL<RegRow<8>>, __VA_ARGS__); break;                               \
-    case 16: hipLaunchKernelGGL(KERNEL<RegRow<16>>, __VA_ARGS__); break;                             \
-    case 24: hipLaunchKernelGGL(KERNEL<RegRow<24>>, __VA_ARGS__); break;                             \
-    default: hipLaunchKernelGGL(KERNEL<GlobalRow>, __VA_ARGS__); break;                              \
+// Calls launch(RowType<Row>{}) with the row type of a vocabulary.
+template <typename T>
+struct RowType {
+  using Row = T;
+};
+template <typename F>
+void with_row(int64_t V, F&& launch) {
+  switch (chunks_for(V)) {
+    case 1: launch(RowType<RegRow<1>>{}); break;
+    case 2: launch(RowType<RegRow<2>>{}); break;
+    case 4: launch(RowType<RegRow<4>>{}); break;
+    case 8: launch(RowType<RegRow<8>>{}); break;
+    case 16: launch(RowType<RegRow<16>>{}); break;
+    case 24: launch(RowType<RegRow<24>>{}); break;
+    default: launch(RowType<GlobalRow>{}); break;
   }
+}
+bool filters(const SideParams& p) { return p.use_p || p.use_k; }
 
 int check_rows(int64_t rows, int64_t V, const void* x) {
   if (rows <= 0 || V <= 0 || !x) return set_error(ASPEC_ERR_INVALID, "sampling needs nonempty bf16 logits");
@@ -1017,8 +1224,13 @@ extern "C" int aspec_sampling_logits_fwd(const void* logits, int64_t rows, int64
   a.out = out;
   a.stats = stats;
   if ((rc = side_params(temperature, top_p, top_k, vocab, &a.px))) return rc;
-  ASPEC_SAMPLING_DISPATCH(sampling_fwd_kernel, chunks_for(vocab), dim3(static_cast<uint32_t>(rows)),
-                          dim3(kSampThreads), 0, static_cast<hipStream_t>(stream), a);
+  const dim3 grid(static_cast<uint32_t>(rows)), block(kSampThreads);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  with_row(vocab, [&](auto type) {
+    using Row = typename decltype(type)::Row;
+    if (filters(a.px)) hipLaunchKernelGGL((sampling_fwd_kernel<Row, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((sampling_fwd_kernel<Row, false>), grid, block, 0, s, a);
+  });
   return check_launch("sampling logits");
 }
 
@@ -1035,8 +1247,11 @@ extern "C" int aspec_sampling_logits_bwd(const void* logits, const float* grad_o
   a.gout = grad_out;
   a.stats = const_cast<float*>(stats);
   a.dx = static_cast<uint16_t*>(grad_logits);
-  ASPEC_SAMPLING_DISPATCH(sampling_bwd_kernel, chunks_for(vocab), dim3(static_cast<uint32_t>(rows)),
-                          dim3(kSampThreads), 0, static_cast<hipStream_t>(stream), a);
+  with_row(vocab, [&](auto type) {
+    using Row = typename decltype(type)::Row;
+    hipLaunchKernelGGL(sampling_bwd_kernel<Row>, dim3(static_cast<uint32_t>(rows)), dim3(kSampThreads), 0,
+                       static_cast<hipStream_t>(stream), a);
+  });
   return check_launch("sampling logits backward");
 }
 
@@ -1062,8 +1277,13 @@ extern "C" int aspec_sampled_l1_fwd(const void* logits, const void* teacher, con
   a.flags = status_flags;
   if ((rc = side_params(draft_temperature, draft_top_p, draft_top_k, vocab, &a.px))) return rc;
   if ((rc = side_params(target_temperature, target_top_p, target_top_k, vocab, &a.py))) return rc;
-  ASPEC_SAMPLING_DISPATCH(sampled_l1_fwd_kernel, chunks_for(vocab), dim3(static_cast<uint32_t>(rows)),
-                          dim3(kSampThreads), 0, static_cast<hipStream_t>(stream), a);
+  const dim3 grid(static_cast<uint32_t>(rows)), block(kSampThreads);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  with_row(vocab, [&](auto type) {
+    using Row = typename decltype(type)::Row;
+    if (filters(a.px) || filters(a.py)) hipLaunchKernelGGL((sampled_l1_fwd_kernel<Row, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((sampled_l1_fwd_kernel<Row, false>), grid, block, 0, s, a);
+  });
   return check_launch("sampled L1 forward");
 }
 

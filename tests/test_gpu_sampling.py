@@ -110,6 +110,55 @@ def test_boundary_bin_edges(gpu, vocab, ties):
     assert int(torch.isfinite(sampling_logits(x[:1], (1.0, 0.5, -1))).sum()) == keep
 
 
+def _flat_rows(gpu, vocab, seed):
+    """Rows whose boundary lies among more tokens than a list holds: close values around zero and around
+    24 (bf16 steps of several bins), equal values alone and below outliers, and masked ones with
+    fewer live tokens than top_k (-inf, and a finite value within and beyond the open bin)."""
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    r = torch.randn(8, vocab, device=gpu, generator=g)
+    r[0] *= 0.01
+    r[1] *= 0.3
+    r[2] += 24
+    r[3] = 1.5
+    r[4] = torch.where(r[4] > 2, r[4] + 3, -1.0)
+    live = torch.arange(vocab, device=gpu) % (vocab // 40) == 7
+    for i, masked in ((5, -torch.inf), (6, -30.0), (7, -1e30)):
+        r[i] = torch.where(live, r[i], masked)
+    return r.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("vocab", [2049, 4096, 8193, 32000, 98304, 151937, 300000])
+def test_flat_rows(gpu, vocab):
+    """The search over a row's keys, as test_sampling_logits_bitwise; top-p ending before, in and after
+    top-k's boundary."""
+    x = _flat_rows(gpu, vocab, vocab)
+    xn = _np(x)
+    for sampling in ((1.0, 0.9, -1), (1.2, 0.5, -1), (1.0, 1.0, 50), (0.7, 0.9, 2000), (1.0, 0.05, vocab // 2),
+                     (1.0, 0.999, vocab // 2), (3.0, 1.0, vocab - 1)):
+        got = sampling_logits(x, sampling).cpu()
+        want = torch.from_numpy(S.sampling_logits(xn, sampling).astype(np.float32))
+        margin = S.top_p_margin(xn, sampling)
+        for r in range(x.shape[0]):
+            diff = got[r] != want[r]
+            n = int(diff.sum())
+            assert n == 0 or (margin[r] < 1e-7 and n == 1), (sampling, r, n, margin[r])
+
+
+@pytest.mark.parametrize("vocab", [4096, 32000, 151937])
+def test_sampled_l1_of_flat_rows(gpu, vocab):
+    x = _flat_rows(gpu, vocab, 31).requires_grad_()
+    y = _flat_rows(gpu, vocab, 32)[[2, 0, 1, 3, 5, 4, 7, 6]]
+    target, draft = (0.9, 0.8, -1), (1.0, 0.6, 1500)
+    l1 = compiled_l1_from_logits(x, y, target, draft)
+    (grad,) = torch.autograd.grad(l1.sum(), x)
+    xn, yn = _np(x.detach()), _np(y)
+    ok = np.minimum(S.top_p_margin(xn, draft), S.top_p_margin(yn, target)) >= 1e-7
+    assert ok.sum() >= 5
+    ref, ref_g = S.sampled_l1(xn, yn, target, draft), S.sampled_l1_grad(xn, yn, np.ones(8), target, draft)
+    torch.testing.assert_close(l1.detach().double().cpu()[ok], torch.from_numpy(ref[ok]), atol=2e-6, rtol=2e-5)
+    torch.testing.assert_close(grad.double().cpu()[ok], torch.from_numpy(ref_g[ok]), atol=2e-5, rtol=0.02)
+
+
 @pytest.mark.parametrize("vocab", [17, 8192, 32000, 98304, 151936])
 @pytest.mark.parametrize("top_p", [1 - 2**-24, 1 - 7 * 2**-24, 1 - 2**-17, 0.99999])
 def test_top_p_in_the_last_digits(gpu, vocab, top_p):
