@@ -118,7 +118,9 @@ __device__ __forceinline__ RowCtx ctx_of(const SideStats& s) {
   return RowCtx{s.m, s.rcp_t, (s.flags & kFlagTemp) != 0};
 }
 // A row's support as the passes test it: kept iff the sort value is above `bound`, or equal (-0
-// equals +0) at an index <= last. A row without a filter has bound -inf and every index.
+// equals +0) at an index <= last. A row without a filter has bound -inf and every index. A sort value
+// that is NaN (0 times the infinite reciprocal of a temperature below 2^-128) is kept, so the NaN
+// shows in the result.
 struct Support {
   float bound;
   int32_t last;
@@ -128,7 +130,7 @@ __device__ __forceinline__ Support support_of(const SideStats& s) {
 }
 // branch-free: evaluated for every token of a pass
 __device__ __forceinline__ bool kept(const Support& s, float ord, int32_t idx) {
-  return (ord > s.bound) | ((ord == s.bound) & (idx <= s.last));
+  return !(ord < s.bound) & ((ord != s.bound) | (idx <= s.last));
 }
 // probability of a token after filtering (0 outside the support)
 __device__ __forceinline__ float prob(const Support& s, const RowCtx& c, float zinv, uint32_t h, int32_t idx) {

@@ -223,6 +223,21 @@ def test_sampled_l1_matches_oracle(gpu, vocab, target, draft):
     torch.testing.assert_close(torch.from_numpy(got_g), torch.from_numpy(ref_g[ok]), atol=2e-5, rtol=0.02)
 
 
+@pytest.mark.parametrize("vocab", [17, 32000, 151936])
+def test_temperature_below_its_reciprocal(gpu, vocab):
+    """A temperature whose fp32 reciprocal is infinite: 0 * inf = NaN at the maximum, as in the
+    reference's scaled values, in the filtered logits, the L1 and the gradient."""
+    x = _rows(gpu, 4, vocab, vocab)[:3]
+    tiny = (1e-39, 1.0, -1)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = torch.from_numpy(S.sampling_logits(_np(x), tiny).astype(np.float32))
+    torch.testing.assert_close(sampling_logits(x, tiny).cpu(), want, atol=0, rtol=0, equal_nan=True)
+    xin = x.clone().requires_grad_()
+    l1 = compiled_l1_from_logits(xin, x, TARGET, tiny)
+    assert torch.isnan(l1).all()
+    assert torch.isnan(torch.autograd.grad(l1.sum(), xin)[0]).any(-1).all()
+
+
 def test_identical_rows_and_default(gpu):
     x = _rows(gpu, 6, 32000, 8).requires_grad_()
     for sampling in (DRAFT, TARGET, (0.5, 1.0, -1)):
