@@ -35,7 +35,7 @@ COMMON_FLAGS = [
 ]
 # The loss and sampled-L1 kernels must evaluate draft and teacher probabilities (and the
 # forward's and backward's) with identical instruction sequences; contraction into FMAs stays off.
-PER_FILE_FLAGS = {"loss.hip": ["-ffp-contract=off"], "sampling.hip": ["-ffp-contract=off"]}
+PER_FILE_FLAGS = {name: ["-ffp-contract=off"] for name in ("loss.hip", "sampling.hip", "sampled_l1.hip")}
 
 
 def hipcc() -> str:

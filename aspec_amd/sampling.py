@@ -1,4 +1,5 @@
-"""Sampled L1 and the sampling-filtered logits, on the HIP kernels of csrc/sampling.hip.
+"""Sampled L1 and the sampling-filtered logits, on the HIP kernels of csrc/sampled_l1.hip and
+csrc/sampling.hip.
 
 Drop-ins for `aspec.models.ops.loss.sampling_logits` and `compiled_l1_from_logits`
 (aspec/models/ops/loss.py:57-89), the L1 of the DSpark head when `l1_target_sampling` /

@@ -1,5 +1,5 @@
-"""Sampled L1 and sampling_logits on the GPU (csrc/sampling.hip) against the fp64 oracle
-(oracle/sampling.py) on the same bf16 inputs.
+"""Sampled L1 and sampling_logits on the GPU (csrc/sampled_l1.hip, csrc/sampling.hip) against the fp64
+oracle (oracle/sampling.py) on the same bf16 inputs.
 
 * `sampling_logits`: the filtered fp32 values equal the oracle's bit for bit (kept values and the
   -inf positions), on the reference test's sampling cases, rows with heavy ties (bf16 values on a
