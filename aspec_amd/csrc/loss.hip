@@ -756,86 +756,105 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
   }
 }
 
-// dx = g_ce * (p - onehot(t)) + g_l1 * p * centered  (tiled_l1.py:107-127 for the L1 part).
-// Each workgroup pass covers 256 consecutive chunks of eight logits of one row, so the row's
-// statistics, upstream gradients, target and teacher index are wave-uniform and read through the
-// scalar cache; only the logits and dx use the vector memory path (16-byte accesses at any
-// alignment; a row's last, partial chunk goes element by element).
+// dx = g_ce * (p - onehot(t)) + g_l1 * p * centered  (tiled_l1.py:107-127 for the L1 part), of the
+// eight logits of one chunk (16-byte accesses at any alignment; a row's last, partial chunk goes
+// element by element). `row_read` reads what the row's chunks share.
+template <typename Read>
+__device__ __forceinline__ void grad_chunk(const LossArgs& a, int64_t row, int64_t chunk, bool live_chunk,
+                                           const Read& row_read) {
+  const bool has_y = a.y != nullptr;
+  float st[kStats];
+#pragma unroll
+  for (int i = 0; i < kStats; ++i) st[i] = row_read(a.stats + row * kStats + i);
+  const float gl1 = (has_y && a.g_l1) ? row_read(a.g_l1 + row) : 0.f;
+  float gce = 0.f;
+  int64_t tgt = -1;
+  if (a.g_ce) {
+    tgt = row_read(a.target + row);
+    gce = tgt == a.ignore_index ? 0.f : row_read(a.g_ce + row);
+  }
+  int64_t trow = 0;
+  if (has_y) {
+    trow = a.yidx ? row_read(a.yidx + row) : row;
+    if (trow < 0 || trow >= a.trows) trow = -1;
+  }
+  if (!live_chunk) return;
+  // dx = p * (L1 weight of the element's case + g_ce) - g_ce at the target, p = e_x * (1/S_x) with
+  // e = exp2(v log2e - max log2e) (scaled_exp2) as in the forward.
+  const float nmx = neg_scaled_max(st[0]), nmy = neg_scaled_max(st[2]);
+  const float pos = st[4], neg = st[5], zero = st[6];
+  const float k_gt = (2.f * neg + zero) * gl1 + gce;
+  const float k_lt = (-2.f * pos - zero) * gl1 + gce;
+  const float k_eq = (neg - pos) * gl1 + gce;
+  const int64_t col0 = chunk * 8;
+  const uint16_t* xr = a.x + row * a.V;
+  const uint16_t* yr = (has_y && trow >= 0) ? a.y + trow * a.V : nullptr;
+  const int live = static_cast<int>(min(a.V - col0, static_cast<int64_t>(8)));
+  const uint4 xs = live == 8 ? load_chunk(xr + col0) : load_part(xr + col0, live);
+  const uint4 ys = !yr ? make_uint4(0, 0, 0, 0) : live == 8 ? load_chunk(yr + col0) : load_part(yr + col0, live);
+  const uint32_t xw[4] = {xs.x, xs.y, xs.z, xs.w};
+  const uint32_t yw[4] = {ys.x, ys.y, ys.z, ys.w};
+  float d[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = (e & 1) ? __uint_as_float(xw[e >> 1] & 0xffff0000u) : __uint_as_float(xw[e >> 1] << 16);
+    const float p = scaled_exp2(x, nmx) * st[1];
+    float k = gce;  // no teacher: the CE part alone
+    if (has_y) {
+      if (yr) {
+        const float y = (e & 1) ? __uint_as_float(yw[e >> 1] & 0xffff0000u) : __uint_as_float(yw[e >> 1] << 16);
+        const float q = scaled_exp2(y, nmy) * st[3];
+        k = p > q ? k_gt : (p < q ? k_lt : k_eq);
+      } else {
+        k = NAN;  // teacher row out of range
+      }
+    }
+    d[e] = p * k;
+  }
+  // the CE target column (one lane of the row)
+  if (gce != 0.f && tgt >= col0 && tgt < col0 + 8) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (col0 + e == tgt) d[e] -= gce;
+  }
+  uint32_t out[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out[e] = pack_bf16x2(d[2 * e], d[2 * e + 1]);
+  uint16_t* const dr = a.dx + row * a.V + col0;
+  if (live == 8) {
+    store_chunk(dr, make_uint4(out[0], out[1], out[2], out[3]));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+      if (e < live) dr[e] = static_cast<uint16_t>(out[e >> 1] >> ((e & 1) * 16));
+  }
+}
+
+// Each workgroup pass covers 256 consecutive chunks of one row, so the row's statistics, upstream
+// gradients, target and teacher index are wave-uniform and read through the scalar cache; only the
+// logits and dx use the vector memory path.
 constexpr int kBwdThreads = 256;
 
 __global__ void __launch_bounds__(kBwdThreads) loss_bwd_rows_kernel(LossArgs a) {
   const int64_t per_row = (a.V + 7) / 8;
   const int64_t segs_per_row = (per_row + kBwdThreads - 1) / kBwdThreads;
   const int64_t segs = a.rows * segs_per_row;
-  const bool has_y = a.y != nullptr;
   for (int64_t seg = blockIdx.x; seg < segs; seg += gridDim.x) {
     const int64_t row = seg / segs_per_row;
     const int64_t chunk = (seg - row * segs_per_row) * kBwdThreads + threadIdx.x;
-    float st[kStats];
-#pragma unroll
-    for (int i = 0; i < kStats; ++i) st[i] = scalar_read(a.stats + row * kStats + i);
-    const float gl1 = (has_y && a.g_l1) ? scalar_read(a.g_l1 + row) : 0.f;
-    float gce = 0.f;
-    int64_t tgt = -1;
-    if (a.g_ce) {
-      tgt = scalar_read(a.target + row);
-      gce = tgt == a.ignore_index ? 0.f : scalar_read(a.g_ce + row);
-    }
-    int64_t trow = 0;
-    if (has_y) {
-      trow = a.yidx ? scalar_read(a.yidx + row) : row;
-      if (trow < 0 || trow >= a.trows) trow = -1;
-    }
-    if (chunk >= per_row) continue;
-    // dx = p * (L1 weight of the element's case + g_ce) - g_ce at the target, p = e_x * (1/S_x) with
-    // e = exp2(v log2e - max log2e) (scaled_exp2) as in the forward.
-    const float nmx = neg_scaled_max(st[0]), nmy = neg_scaled_max(st[2]);
-    const float pos = st[4], neg = st[5], zero = st[6];
-    const float k_gt = (2.f * neg + zero) * gl1 + gce;
-    const float k_lt = (-2.f * pos - zero) * gl1 + gce;
-    const float k_eq = (neg - pos) * gl1 + gce;
-    const int64_t col0 = chunk * 8;
-    const uint16_t* xr = a.x + row * a.V;
-    const uint16_t* yr = (has_y && trow >= 0) ? a.y + trow * a.V : nullptr;
-    const int live = static_cast<int>(min(a.V - col0, static_cast<int64_t>(8)));
-    const uint4 xs = live == 8 ? load_chunk(xr + col0) : load_part(xr + col0, live);
-    const uint4 ys = !yr ? make_uint4(0, 0, 0, 0) : live == 8 ? load_chunk(yr + col0) : load_part(yr + col0, live);
-    const uint32_t xw[4] = {xs.x, xs.y, xs.z, xs.w};
-    const uint32_t yw[4] = {ys.x, ys.y, ys.z, ys.w};
-    float d[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = (e & 1) ? __uint_as_float(xw[e >> 1] & 0xffff0000u) : __uint_as_float(xw[e >> 1] << 16);
-      const float p = scaled_exp2(x, nmx) * st[1];
-      float k = gce;  // no teacher: the CE part alone
-      if (has_y) {
-        if (yr) {
-          const float y = (e & 1) ? __uint_as_float(yw[e >> 1] & 0xffff0000u) : __uint_as_float(yw[e >> 1] << 16);
-          const float q = scaled_exp2(y, nmy) * st[3];
-          k = p > q ? k_gt : (p < q ? k_lt : k_eq);
-        } else {
-          k = NAN;  // teacher row out of range
-        }
-      }
-      d[e] = p * k;
-    }
-    // the CE target column (one lane of the row)
-    if (gce != 0.f && tgt >= col0 && tgt < col0 + 8) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (col0 + e == tgt) d[e] -= gce;
-    }
-    uint32_t out[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = pack_bf16x2(d[2 * e], d[2 * e + 1]);
-    uint16_t* const dr = a.dx + row * a.V + col0;
-    if (live == 8) {
-      store_chunk(dr, make_uint4(out[0], out[1], out[2], out[3]));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 7; ++e)
-        if (e < live) dr[e] = static_cast<uint16_t>(out[e >> 1] >> ((e & 1) * 16));
-    }
+    grad_chunk(a, row, chunk, chunk < per_row, [](const auto* p) { return scalar_read(p); });
+  }
+}
+
+// Short rows, which would leave most of such a workgroup idle: the chunks of all rows in one sequence,
+// each thread reading its row's statistics.
+__global__ void __launch_bounds__(kBwdThreads) loss_bwd_short_kernel(LossArgs a) {
+  const int64_t per_row = (a.V + 7) / 8;
+  const int64_t chunks = a.rows * per_row;
+  for (int64_t c = static_cast<int64_t>(blockIdx.x) * kBwdThreads + threadIdx.x; c < chunks;
+       c += static_cast<int64_t>(gridDim.x) * kBwdThreads) {
+    const int64_t row = c / per_row;
+    grad_chunk(a, row, c - row * per_row, true, [](const auto* p) { return *p; });
   }
 }
 
@@ -857,6 +876,15 @@ void launch_walk(const LossArgs& a, int cus, hipStream_t s) {
   }
 }
 
+// Rows up to kShortRow logits take one wave each in the two-pass forward: a workgroup's waves would be
+// mostly idle and meet at every reduction. 200000 rows x 9 logits 1165 -> 314 us with 64 instead of 256
+// threads, 20000 x 1001 145 -> 57, 8192 x 2047 72 -> 46; at 64 rows of 4095 it is the slower one,
+// 26 against 23.6 us.
+constexpr int64_t kShortRow = 2048;
+// Rows up to kShortChunks chunks take the backward over all rows' chunks: 200000 rows x 9 logits
+// 171 -> 10 us against a workgroup per row, 65536 x 257 63 -> 27, 20000 x 1001 31 -> 27; 8192 x 2047
+// 25 -> 27.
+constexpr int64_t kShortChunks = 128;
 template <int THREADS>
 void launch_streaming(const LossArgs& a, dim3 grid, hipStream_t s) {
   if (a.y) hipLaunchKernelGGL((loss_fwd_streaming<THREADS, true>), grid, dim3(THREADS), 0, s, a);
@@ -880,6 +908,8 @@ int launch_fwd(const LossArgs& a, hipStream_t s) {
     launch_walk<4>(a, cus, s);
   } else if (vec && a.V <= kWalkThreads * 8 * 8) {
     launch_walk<8>(a, cus, s);
+  } else if (a.V <= kShortRow) {
+    launch_streaming<64>(a, grid, s);
   } else if (a.V <= 8192) {  // one workgroup per row, as many threads as its chunks keep busy
     launch_streaming<256>(a, grid, s);
   } else {
@@ -889,9 +919,13 @@ int launch_fwd(const LossArgs& a, hipStream_t s) {
 }
 
 int launch_bwd(const LossArgs& a, hipStream_t s) {
-  const int64_t segs = a.rows * (((a.V + 7) / 8 + kBwdThreads - 1) / kBwdThreads);
-  const int64_t grid = std::min<int64_t>(segs, 256 * 64);
-  hipLaunchKernelGGL(loss_bwd_rows_kernel, dim3(static_cast<uint32_t>(grid)), dim3(kBwdThreads), 0, s, a);
+  const int64_t per_row = (a.V + 7) / 8;
+  const bool by_row = per_row > kShortChunks;
+  const int64_t blocks = by_row ? a.rows * ((per_row + kBwdThreads - 1) / kBwdThreads)
+                                : (a.rows * per_row + kBwdThreads - 1) / kBwdThreads;
+  const dim3 grid(static_cast<uint32_t>(std::min<int64_t>(blocks, 256 * 64)));
+  if (by_row) hipLaunchKernelGGL(loss_bwd_rows_kernel, grid, dim3(kBwdThreads), 0, s, a);
+  else hipLaunchKernelGGL(loss_bwd_short_kernel, grid, dim3(kBwdThreads), 0, s, a);
   return check_launch("loss backward");
 }
 

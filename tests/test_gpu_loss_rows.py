@@ -1,7 +1,8 @@
 """The two-pass loss forward and the backward at any vocabulary and row alignment (V % 8 != 0, rows
 past the row walk's reach), against the fp64 oracle at the edges of their chunks and steps: fewer
 logits than a chunk, a lone tail, exact multiples of a step (8 x 256 or 512 logits) and one more or
-less, and the 256- to 512-thread border. Bars as in tests/test_gpu_loss.py; the argmax exact."""
+less, and the borders between 64, 256 and 512 threads and between the two backwards. Bars as in
+tests/test_gpu_loss.py; the argmax exact."""
 
 import numpy as np
 import pytest
@@ -13,7 +14,7 @@ from oracle import loss as L
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("vocab", [1, 7, 9, 2047, 2049, 4095, 4097, 8191, 8193, 16383, 32769, 40960, 65537, 152063])
+@pytest.mark.parametrize("vocab", [1, 7, 9, 257, 1017, 1024, 1025, 2047, 2049, 4095, 4097, 8191, 8193, 16383, 32769, 40960, 65537, 152063])
 def test_any_vocabulary(gpu, vocab):
     rows, trows = 5, 3
     g = torch.Generator(device=gpu).manual_seed(vocab)
