@@ -41,16 +41,12 @@ struct LossArgs {
 
 __device__ __forceinline__ float fexp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Block-wide reduction of NVAL floats (sum or max), result broadcast to every thread.
-template <int NVAL, bool MAX>
+// Block-wide sums of NVAL floats, broadcast to every thread.
+template <int NVAL>
 __device__ __forceinline__ void block_reduce(float (&v)[NVAL], float* scratch) {
 #pragma unroll
-  for (int i = 0; i < NVAL; ++i) {
-    for (int off = 32; off > 0; off >>= 1) {
-      const float o = __shfl_xor(v[i], off);
-      v[i] = MAX ? fmaxf(v[i], o) : v[i] + o;
-    }
-  }
+  for (int i = 0; i < NVAL; ++i)
+    for (int off = 32; off > 0; off >>= 1) v[i] += __shfl_xor(v[i], off);
   const int wave = threadIdx.x >> 6;
   const int nwaves = blockDim.x >> 6;
   __syncthreads();
@@ -62,7 +58,7 @@ __device__ __forceinline__ void block_reduce(float (&v)[NVAL], float* scratch) {
 #pragma unroll
   for (int i = 0; i < NVAL; ++i) {
     float r = scratch[i * 32];
-    for (int w = 1; w < nwaves; ++w) r = MAX ? fmaxf(r, scratch[i * 32 + w]) : r + scratch[i * 32 + w];
+    for (int w = 1; w < nwaves; ++w) r += scratch[i * 32 + w];
     v[i] = r;
   }
 }
@@ -557,12 +553,12 @@ loss_fwd_persistent(LossArgs args) {
 // A chunk starts at a multiple of eight logits of its row, so at any 2-byte address when V % 8 != 0:
 // its load is one 16-byte access all the same (global memory takes any alignment on this target).
 //
-// What bounds it: both passes' reads. A 151936-token row and its teacher are 608 KB, more than a CU's
-// registers and LDS hold, so they are read twice; at 2048 rows against 1024 teacher rows the two
-// passes move 2.5 GB past the L2 in 395-420 us (6 TB/s; the previous kernel, element loads in three
-// passes, took 1467 us). Per logit pair pass 1 costs about 12 VALU slots and pass 2 16. Kept: two
-// chunks in flight per thread (one or three measured the same) and 512 threads (1024: 483 us at
-// 2048 rows and no faster at 64 rows; 256: the same at 2048 rows, 57 against 41 us at 64).
+// What bounds it: the VALU and both passes' reads, nearly alike. A 151936-token row and its teacher are
+// 608 KB, more than a CU's registers and LDS hold, so they are read twice; at 2048 rows against 1024
+// teacher rows the two passes read 2.43 GB past the L2 in 376 us (6.5 TB/s), with 34 VALU instructions
+// per logit pair busy 0.90 of the time (element loads in three passes took 1467 us). Kept: two chunks
+// in flight per thread (one or three measured the same) and 512 threads (1024: 483 us at 2048 rows
+// and no faster at 64 rows; 256: the same at 2048 rows, 57 against 41 us at 64).
 template <int THREADS, bool HAS_Y>
 __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
   __shared__ float scratch[4 * 32];
@@ -735,7 +731,7 @@ __global__ void __launch_bounds__(THREADS) loss_fwd_streaming(LossArgs a) {
       acc[2] += d < 0.f ? p : 0.f;
       acc[3] += (d > 0.f) | (d < 0.f) ? 0.f : p;
     }
-    block_reduce<4, false>(acc, scratch);
+    block_reduce<4>(acc, scratch);
   }
   if (tid == 0) {
     // less the rounding of the offset, which all of S_x carries

@@ -89,7 +89,7 @@ def test_tie_groups_exact(gpu, vocab):
         assert kept[:, :n].all() and not kept[:, n:].any()
 
 
-@pytest.mark.parametrize("vocab", [4097, 32000, 70001, 151936])
+@pytest.mark.parametrize("vocab", [4101, 32000, 70001, 151936])
 @pytest.mark.parametrize("ties", [2047, 2048, 2049])
 def test_boundary_bin_edges(gpu, vocab, ties):
     """The boundary in a bin of as many tokens as the list holds, one fewer and one more, and in the
@@ -97,6 +97,7 @@ def test_boundary_bin_edges(gpu, vocab, ties):
     Filters by count only, or with the boundary's margin far above rounding: exact."""
     x = torch.full((2, vocab), -100.0, device=gpu)
     x[:, 3::2][:, :ties] = 1.0  # one bin: `ties` equal tokens, below three larger ones
+    assert int((x[0] == 1.0).sum()) == ties
     x[:, :3] = 3.0
     x[1, 5::7] = -torch.inf
     x = x.to(torch.bfloat16)
