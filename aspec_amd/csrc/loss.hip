@@ -555,8 +555,8 @@ loss_fwd_persistent(LossArgs args) {
 //
 // What bounds it: the VALU and both passes' reads, nearly alike. A 151936-token row and its teacher are
 // 608 KB, more than a CU's registers and LDS hold, so they are read twice; at 2048 rows against 1024
-// teacher rows the two passes read 2.43 GB past the L2 in 376 us (6.5 TB/s), with 34 VALU instructions
-// per logit pair busy 0.90 of the time (element loads in three passes took 1467 us). Kept: two chunks
+// teacher rows the two passes read 2.43 GB past the L2 in 375 us (6.5 TB/s), with 34 VALU instructions
+// per logit pair busy 0.92 of the time (element loads in three passes took 1467 us). Kept: two chunks
 // in flight per thread (one or three measured the same) and 512 threads (1024: 483 us at 2048 rows
 // and no faster at 64 rows; 256: the same at 2048 rows, 57 against 41 us at 64).
 template <int THREADS, bool HAS_Y>
